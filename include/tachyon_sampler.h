@@ -297,17 +297,17 @@ int tsm_json_mask(void* stream, const tsm_vocab* vocab, const tsm_json_state* st
  * with the per-state reuse the reference's probing has no need of.
  *
  * tsm_json_masks_create allocates the set on `device` (GPU memory:
- * capacity * ceil(ceil(usable / 32) / 64) * 256 bytes, plus about 2 * 44
- * bytes per row of staging in pinned host memory, which the kernels read over
- * the bus); `capacity` 0 keeps no
+ * capacity * ceil(ceil(usable / 32) / 64) * 256 bytes plus about 32 bytes per
+ * row, and about 2 * 40 bytes per row of staging in pinned host memory, which
+ * one kernel of a call reads over the bus); `capacity` 0 keeps no
  * masks between calls (rows sharing a state within a call still share one
  * evaluation).  NULL on failure, with the reason in err.
  *
  * tsm_json_masks_fill: `states` is a HOST array of `rows` (<= max_rows)
  * states, as tsm_json_advance keeps them; `mask` (device) gets one row per
  * state, words [0, ceil(usable / 32)) of each written.  `stats` (may be NULL)
- * receives the call's counts.  Queued on `stream`: at most one evaluation
- * launch and one copy launch.  The call waits on the host only for the
+ * receives the call's counts.  Queued on `stream`: one copy launch and at
+ * most one evaluation launch.  The call waits on the host only for the
  * launches of the call before the last one (the staging alternates between
  * two halves).  The slots are tied to the
  * vocabulary's device pointers and n_tokens: a call with other ones empties

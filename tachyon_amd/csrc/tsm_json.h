@@ -217,5 +217,277 @@ __host__ __device__ inline bool accepts(tsm_json_state s, const uint8_t* bytes, 
     return true;
 }
 
+// ---- the automaton as a table -----------------------------------------------
+// step() with its finite part written out: a flat state per (state, aux,
+// literal position), 30 byte classes, and per pair the next flat state and an
+// action on the counters (stack, depth, whitespace run, number length).  A GPU
+// lane then takes one table word and a few predicated operations a byte where
+// step() takes a chain of data-dependent branches, which a wave of different
+// tokens walks one after another.
+enum : uint32_t {  // byte classes: bytes step() never tells apart
+    C_CTRL = 0, C_SPACE, C_BLANK /* \t \n \r */, C_QUOTE, C_BSLASH, C_SLASH, C_LBRACE, C_RBRACE, C_LBRACK, C_RBRACK,
+    C_COMMA, C_COLON, C_MINUS, C_PLUS, C_DOT, C_0, C_19, C_e, C_E, C_a, C_b, C_f, C_HEX /* c d A B C D F */, C_n,
+    C_r, C_t, C_u, C_l, C_s, C_TEXT /* the rest, >= 0x20 */, C_COUNT
+};
+constexpr uint32_t kClasses = 32;  // table row length
+static_assert(C_COUNT <= kClasses, "byte classes fit a table row");
+
+constexpr uint32_t byte_class(uint32_t b) {
+    switch (b) {
+        case ' ': return C_SPACE;
+        case '\t': case '\n': case '\r': return C_BLANK;
+        case '"': return C_QUOTE;
+        case '\\': return C_BSLASH;
+        case '/': return C_SLASH;
+        case '{': return C_LBRACE;
+        case '}': return C_RBRACE;
+        case '[': return C_LBRACK;
+        case ']': return C_RBRACK;
+        case ',': return C_COMMA;
+        case ':': return C_COLON;
+        case '-': return C_MINUS;
+        case '+': return C_PLUS;
+        case '.': return C_DOT;
+        case '0': return C_0;
+        case 'e': return C_e;
+        case 'E': return C_E;
+        case 'a': return C_a;
+        case 'b': return C_b;
+        case 'f': return C_f;
+        case 'c': case 'd': case 'A': case 'B': case 'C': case 'D': case 'F': return C_HEX;
+        case 'n': return C_n;
+        case 'r': return C_r;
+        case 't': return C_t;
+        case 'u': return C_u;
+        case 'l': return C_l;
+        case 's': return C_s;
+        default: return b >= '1' && b <= '9' ? C_19 : b < 0x20 ? C_CTRL : C_TEXT;
+    }
+}
+// Text bytes: what passes inside a string whatever else is around.
+constexpr uint32_t kTextClasses =
+    ~((1u << C_CTRL) | (1u << C_BLANK) | (1u << C_QUOTE) | (1u << C_BSLASH)) & ((1u << C_COUNT) - 1u);
+
+enum : uint32_t {  // flat states
+    F_VALUE = 0, F_ARRAY_START, F_OBJECT_START, F_KEY, F_COLON, F_AFTER, F_DONE, F_ROOT /* a value at depth 0 */,
+    F_STR = 8,            // + 6 * key + (0: text, 1: escape, 1 + h: h hex digits left)
+    F_NUM = F_STR + 12,   // + number part
+    F_LIT = F_NUM + 8,    // + kLitBase[word] + bytes matched - 1
+    F_OTHER = F_LIT + 10, // none of these (not a state an accepted text leaves): stepped by step()
+    F_COUNT = F_OTHER
+};
+// A walk keeps the containers as a shift register (the innermost in bit 0) and
+// its three counters in one word, each biased so that passing its limit sets
+// its top bit.
+constexpr uint32_t kWsBias = 127u - kMaxWhitespace, kLenBias = 127u - kMaxNumber, kDepthBias = 127u - kMaxDepth;
+constexpr uint32_t kLimits = 0x00808080u;  // whitespace, number length << 8, depth << 16
+constexpr uint32_t kDepth1 = 1u << 16;
+
+// A table entry: word x, the next flat state's row (flat * kClasses) and flags;
+// word y, what is added to the counters once their low (x >> W_RESET) & 31 bits
+// are cleared.
+enum : uint32_t {
+    W_ROW = 0x7FFu,
+    W_USED = 1u << 11,     // the byte is used up (else it is taken again, after a number's end)
+    W_OBJ = 1u << 12,      // a container opens or closes: an object (else an array)
+    W_OPEN = 1u << 13,
+    W_CLOSE = 1u << 14,
+    W_END = 1u << 15,      // a value ended: what follows depends on the depth
+    W_COMMA = 1u << 16,    // what follows depends on the container
+    W_REJECT = 1u << 17,
+    W_RESET = 18
+};
+struct Entry {
+    uint32_t x, y;
+};
+constexpr Entry entry(uint32_t flat, uint32_t flags, uint32_t add = 0, uint32_t reset = 0) {
+    return Entry{flat * kClasses | flags | reset << W_RESET, add};
+}
+// the steps a byte can make
+constexpr Entry e_reject(uint32_t f) { return entry(f, W_REJECT | W_USED); }
+constexpr Entry e_go(uint32_t next) { return entry(next, W_USED); }
+constexpr Entry e_blank(uint32_t f) { return entry(f, W_USED, 1u); }
+// a structural byte ends the whitespace run
+constexpr Entry e_mark(uint32_t next, uint32_t flags = 0, uint32_t add = 0) {
+    return entry(next, flags | W_USED, kWsBias + add, 8u);
+}
+constexpr Entry e_open(bool obj) {
+    return obj ? e_mark(F_OBJECT_START, W_OPEN | W_OBJ, kDepth1) : e_mark(F_ARRAY_START, W_OPEN, kDepth1);
+}
+constexpr Entry e_close(bool obj) { return e_mark(0, W_CLOSE | W_END | (obj ? W_OBJ : 0u), 0u - kDepth1); }
+constexpr Entry e_value_end() { return entry(0, W_END | W_USED); }
+constexpr Entry e_number(uint32_t part) {
+    return entry(F_NUM + part, W_USED, kWsBias | (kLenBias + 1u) << 8, 16u);
+}
+constexpr Entry e_digit(uint32_t part) { return entry(F_NUM + part, W_USED, 1u << 8); }
+constexpr Entry e_number_end() { return entry(0, W_END); }
+
+constexpr uint32_t lit_base(uint32_t word) { return word == 0 ? 0u : word == 1 ? 3u : 7u; }
+constexpr uint32_t lit_class(uint32_t word, uint32_t at) {
+    constexpr uint8_t w[3][5] = {{C_t, C_r, C_u, C_e, 0}, {C_f, C_a, C_l, C_s, C_e}, {C_n, C_u, C_l, C_l, 0}};
+    return w[word][at];
+}
+
+// The next number part after a byte of class c, 0xFF when none (number_next).
+constexpr uint32_t number_class_next(uint32_t n, uint32_t c) {
+    const bool d = c == C_0 || c == C_19, ex = c == C_e || c == C_E;
+    switch (n) {
+        case N_MINUS: return c == C_0 ? uint32_t(N_ZERO) : (d ? uint32_t(N_INT) : 0xFFu);
+        case N_ZERO: return c == C_DOT ? uint32_t(N_DOT) : ex ? uint32_t(N_EXP) : 0xFFu;
+        case N_INT: return c == C_DOT ? uint32_t(N_DOT) : d ? uint32_t(N_INT) : ex ? uint32_t(N_EXP) : 0xFFu;
+        case N_DOT: return d ? uint32_t(N_FRAC) : 0xFFu;
+        case N_FRAC: return d ? uint32_t(N_FRAC) : ex ? uint32_t(N_EXP) : 0xFFu;
+        case N_EXP: return (c == C_PLUS || c == C_MINUS) ? uint32_t(N_EXPSIGN) : d ? uint32_t(N_EXPDIGITS) : 0xFFu;
+        default: return d ? uint32_t(N_EXPDIGITS) : 0xFFu;  // N_EXPSIGN, N_EXPDIGITS
+    }
+}
+
+constexpr Entry table_entry(uint32_t f, uint32_t c) {
+    if (f >= F_LIT) {
+        const uint32_t k = f - F_LIT, word = k < 3u ? 0u : k < 7u ? 1u : 2u;
+        const uint32_t at = k - lit_base(word) + 1u, n = word == 1u ? 5u : 4u;
+        if (c != lit_class(word, at)) return e_reject(f);
+        return at + 1u == n ? e_value_end() : e_go(f + 1u);
+    }
+    if (f >= F_NUM) {
+        const uint32_t part = f - F_NUM, next = number_class_next(part, c);
+        if (next != 0xFFu) return e_digit(next);
+        const bool whole = part == N_ZERO || part == N_INT || part == N_FRAC || part == N_EXPDIGITS;
+        return whole ? e_number_end() : e_reject(f);
+    }
+    if (f >= F_STR) {
+        const uint32_t key = (f - F_STR) / 6u, sub = (f - F_STR) % 6u, text = F_STR + 6u * key;
+        if (sub >= 2u) {
+            const bool hex = c == C_0 || c == C_19 || c == C_a || c == C_b || c == C_e || c == C_f || c == C_E || c == C_HEX;
+            return hex ? e_go(sub == 2u ? text : f - 1u) : e_reject(f);
+        }
+        if (sub == 1u) {
+            if (c == C_u) return e_go(text + 5u);
+            const bool esc = c == C_QUOTE || c == C_BSLASH || c == C_SLASH || c == C_b || c == C_f || c == C_n ||
+                             c == C_r || c == C_t;
+            return esc ? e_go(text) : e_reject(f);
+        }
+        if (c == C_QUOTE) return key ? e_go(F_COLON) : e_value_end();
+        if (c == C_BSLASH) return e_go(f + 1u);
+        return ((kTextClasses >> c) & 1u) ? e_go(f) : e_reject(f);
+    }
+    if (f == F_DONE) return e_reject(f);
+    if (c == C_SPACE || c == C_BLANK) return e_blank(f);
+    switch (f) {
+        case F_ROOT: return c == C_LBRACE ? e_open(true) : e_reject(f);
+        case F_OBJECT_START:
+            if (c == C_RBRACE) return e_close(true);
+            return c == C_QUOTE ? e_mark(F_STR + 6u) : e_reject(f);
+        case F_KEY: return c == C_QUOTE ? e_mark(F_STR + 6u) : e_reject(f);
+        case F_COLON: return c == C_COLON ? e_mark(F_VALUE) : e_reject(f);
+        case F_AFTER:
+            if (c == C_COMMA) return e_mark(F_VALUE, W_COMMA);
+            if (c == C_RBRACE) return e_close(true);
+            return c == C_RBRACK ? e_close(false) : e_reject(f);
+        default: break;  // F_VALUE, F_ARRAY_START
+    }
+    if (f == F_ARRAY_START && c == C_RBRACK) return e_close(false);
+    switch (c) {
+        case C_LBRACE: return e_open(true);
+        case C_LBRACK: return e_open(false);
+        case C_QUOTE: return e_mark(F_STR);
+        case C_MINUS: return e_number(N_MINUS);
+        case C_0: return e_number(N_ZERO);
+        case C_19: return e_number(N_INT);
+        case C_t: return e_mark(F_LIT + lit_base(0));
+        case C_f: return e_mark(F_LIT + lit_base(1));
+        case C_n: return e_mark(F_LIT + lit_base(2));
+        default: return e_reject(f);
+    }
+}
+
+constexpr uint32_t kNotText = 0x80u;
+
+struct Tables {
+    Entry next[F_COUNT * kClasses];
+    // per flat state: the classes a token may start with (F_OTHER: all); a
+    // number that can end hands the byte to what follows a value
+    uint32_t first[F_COUNT + 1];
+    uint8_t cls[256];  // a byte's class, with kNotText
+};
+constexpr Tables make_tables() {
+    Tables t{};
+    for (uint32_t f = 0; f < F_COUNT; f++)
+        for (uint32_t c = 0; c < kClasses; c++) {
+            const Entry e = c < C_COUNT ? table_entry(f, c) : e_reject(f);
+            t.next[f * kClasses + c] = e;
+            if (!(((e.x & W_USED) ? e : table_entry(F_AFTER, c)).x & W_REJECT)) t.first[f] |= 1u << c;
+        }
+    t.first[F_OTHER] = 0xFFFFFFFFu;
+    for (uint32_t b = 0; b < 256u; b++) t.cls[b] = static_cast<uint8_t>(byte_class(b) | (((kTextClasses >> byte_class(b)) & 1u) ? 0u : kNotText));
+    return t;
+}
+
+// A state's flat state.
+__host__ __device__ inline uint32_t flat_of(const tsm_json_state& s) {
+    if (s.depth > kMaxDepth || s.whitespace > kMaxWhitespace) return F_OTHER;
+    switch (s.state) {
+        case JS_VALUE: return s.depth ? uint32_t(F_VALUE) : uint32_t(F_ROOT);
+        case JS_DONE: return F_DONE;
+        case JS_STR: {
+            const uint32_t key = s.aux & 1u, esc = (s.aux >> 1) & 1u, hex = s.aux >> 2;
+            if (hex > 4u || (hex && esc) || (key && s.depth == 0)) return F_OTHER;
+            return F_STR + 6u * key + (hex ? 1u + hex : esc);
+        }
+        case JS_NUMBER: return s.aux <= N_EXPDIGITS && s.len <= kMaxNumber ? F_NUM + s.aux : uint32_t(F_OTHER);
+        case JS_LITERAL:
+            if (s.aux > 2u || s.len == 0 || s.len >= (s.aux == 1u ? 5u : 4u)) return F_OTHER;
+            return F_LIT + lit_base(s.aux) + s.len - 1u;
+        default:
+            if (s.depth == 0 || s.state > JS_DONE) return F_OTHER;
+            return s.state;  // JS_ARRAY_START .. JS_AFTER: the flat states have the same numbers
+    }
+}
+static_assert(int(F_ARRAY_START) == int(JS_ARRAY_START) && int(F_OBJECT_START) == int(JS_OBJECT_START) &&
+                  int(F_KEY) == int(JS_KEY) && int(F_COLON) == int(JS_COLON) && int(F_AFTER) == int(JS_AFTER),
+              "structural states keep their numbers");
+
+// A state with flat state f without what no later byte can depend on: aux and
+// len outside strings, numbers and literals (what they left behind), stack
+// levels above the depth, everything of a closed object.
+__host__ __device__ inline void forget(tsm_json_state* s, uint32_t f) {
+    s->pad[0] = s->pad[1] = s->pad[2] = 0;
+    if (f == F_OTHER) return;
+    if (f < F_STR) s->aux = 0;
+    if (f < F_NUM) s->len = 0;
+    s->stack &= s->depth < kMaxDepth ? (1u << s->depth) - 1u : 0xFFFFFFFFu;
+    if (f == F_DONE) {
+        s->stack = 0;
+        s->depth = s->whitespace = 0;
+    }
+}
+
+// A walk through a token's byte classes.
+struct Walk {
+    uint32_t row, stack, count;
+};
+__host__ __device__ inline Walk walk_of(const tsm_json_state& s, uint32_t f) {
+    Walk w{f * kClasses, 0u, (s.whitespace + kWsBias) | (f >= F_NUM && f < F_LIT ? s.len + kLenBias : 0u) << 8 |
+                                 (s.depth + kDepthBias) << 16};
+    for (uint32_t i = 0; i < s.depth; i++) w.stack = w.stack << 1 | ((s.stack >> i) & 1u);
+    return w;
+}
+// One step by table entry e = next[row + (class & 31)]; false when the byte is
+// rejected.  (A container closes only inside one: at depth 0 no flat state has
+// a closing step.)
+__host__ __device__ inline bool step_entry(Walk& w, Entry e) {
+    const uint32_t obj = (e.x / W_OBJ) & 1u, top = w.stack & 1u;
+    bool bad = (e.x & W_REJECT) != 0u;
+    bad |= (e.x & W_CLOSE) && top != obj;
+    w.count = (w.count & (0xFFFFFFFFu << ((e.x >> W_RESET) & 31u))) + e.y;
+    bad |= (w.count & kLimits) != 0u;
+    w.stack = (e.x & W_OPEN) ? w.stack << 1 | obj : (e.x & W_CLOSE) ? w.stack >> 1 : w.stack;
+    uint32_t row = e.x & W_ROW;
+    if (e.x & W_END) row = (w.count >> 16) == kDepthBias ? F_DONE * kClasses : F_AFTER * kClasses;
+    if ((e.x & W_COMMA) && top) row = F_KEY * kClasses;
+    w.row = row;
+    return !bad;
+}
+
 }  // namespace json
 }  // namespace tsm
