@@ -49,8 +49,8 @@ constexpr uint32_t kOffECnt = kOffE;                     // u32[kNB] candidates 
 constexpr uint32_t kOffEMass = kOffECnt + kNB * 4;       // f64[kNB] approximate masses; after planning:
 constexpr uint32_t kOffESStart = kOffEMass;              //   f32[kNB] total's fold value at each bin start
 constexpr uint32_t kOffEPStart = kOffEMass + kNB * 4;    //   u32[kNB] candidates before each bin
-constexpr uint32_t kOffELay = kOffEMass + kNB * 8;       // u32[kNB] candidates before each coarse bin
-constexpr uint32_t kOffEPlan = kOffELay + kNB * 4;       // u32[kNB] grid plans
+constexpr uint32_t kOffELay = kOffEMass + kNB * 8;       // u32[kNB + 1] weight before each coarse bin, and past the last
+constexpr uint32_t kOffEPlan = kOffELay + (kNB + 2) * 4;       // u32[kNB] grid plans
 constexpr uint32_t kOffESum = kOffEPlan + kNB * 4;       // u32[4][kNB] grid sums
 constexpr uint32_t kOffETie = kOffESum + 4 * kNB * 4;    // u32[4 * kNB / 32] sums with a tie or invalid
 constexpr uint32_t kOffETieB = kOffETie + kNB * 4 / 8;   // u32[4 * kNB / 32] sums invalid (or two ties)
@@ -127,6 +127,7 @@ enum : uint32_t {  // e_sc() words
     SC_OVF = 12,    // census table full
     SC_CMIN = 13,   // smallest candidate value's total key
     SC_TIED = 14,   // walk: a bin sum it added holds a tie
+    SC_FILED = 15,  // elements filed for the census
 };
 
 // Grid plan of a bin, one byte per fold for the lower grid's binade (+128)
@@ -135,6 +136,7 @@ enum : uint32_t {
     PF_TWO_S = 1u << 24, PF_TWO_R = 1u << 25, PF_TWO_A = 1u << 26,
     PF_MUST_S = 1u << 27, PF_MUST_R = 1u << 28, PF_MUST_A = 1u << 29,
     PF_R = 1u << 30,  // the draw may reach this bin
+    PF_REQ = 1u << 31,  // requested of the census (census_clear)
 };
 enum : int { FK_S = 0, FK_A = 1, FK_R = 2 };  // total (and the kept mass), acc, the draw
 enum : uint32_t { SL_S0 = 0, SL_S1 = 1, SL_R0 = 2, SL_R1 = 3 };  // acc reuses slots 0 and 1
@@ -189,21 +191,13 @@ __device__ __forceinline__ uint32_t grid_term(float tau, int e, uint32_t* fl = n
     return static_cast<uint32_t>(k) + (fr > 0.5f ? 1u : 0u);
 }
 
-__device__ __forceinline__ uint64_t wave_incl_scan64(uint64_t v, uint32_t lane) {
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-        const uint64_t w = __shfl_up(v, static_cast<unsigned>(o), kWave);
-        if (lane >= static_cast<uint32_t>(o)) v += w;
-    }
-    return v;
+// thr in units of 2^g, rounded up; at most 2^31 (past every fold value's units).
+__device__ __forceinline__ uint32_t grid_ceil(float thr, int g) {
+    return static_cast<uint32_t>(fminf(ceilf(ldexpf(thr, -g)), 2147483648.0f));
 }
+
 __device__ __forceinline__ uint32_t first_lane(uint64_t mask) {
     return mask ? static_cast<uint32_t>(__builtin_ctzll(mask)) : 64u;
-}
-__device__ __forceinline__ uint64_t wave_read64(uint64_t v, uint32_t lane) {
-    const uint32_t lo = wave_read(static_cast<uint32_t>(v), lane);
-    const uint32_t hi = wave_read(static_cast<uint32_t>(v >> 32), lane);
-    return (static_cast<uint64_t>(hi) << 32) | lo;
 }
 
 // ---- bins -----------------------------------------------------------------------
@@ -233,20 +227,22 @@ struct FBins {
     VBins vb;
     float scale;
     uint32_t cr[kCrowd];  // crowded coarse bins laid out from their own sub-histogram (kNoBin: none)
+    // (branchless: fmaxf and fminf take a NaN to the other bound)
     __device__ __forceinline__ float frac(float y, uint32_t c) const {
-        const float fr = vb.pos(y) - static_cast<float>(c);
-        return fr > 0.0f ? (fr < 1.0f ? fr : 1.0f) : 0.0f;
+        return fminf(fmaxf(vb.pos(y) - static_cast<float>(c), 0.0f), 1.0f);
     }
     __device__ __forceinline__ uint32_t bin(float y) const {
         const uint32_t c = vb.bin(y);
         if (scale == 0.0f) return c;
-        const uint32_t c0 = e_lay()[c], c1 = c + 1u < kNB ? e_lay()[c + 1u] : c0 + (kNB - 1u);
+        const uint32_t c0 = e_lay()[c], c1 = e_lay()[c + 1u];
         float fr = frac(y, c);
+        if (cr[0] != kNoBin) {  // any bin crowded at all (the same for the whole workgroup)
 #pragma unroll
-        for (uint32_t s = 0; s < kCrowd; s++)
-            if (c == cr[s]) fr = crowd_frac(e_cdf(s), fr);
+            for (uint32_t s = 0; s < kCrowd; s++)
+                if (c == cr[s]) fr = crowd_frac(e_cdf(s), fr);
+        }
         const float v = (static_cast<float>(c0) + fr * static_cast<float>(c1 - c0)) * scale;
-        return v >= static_cast<float>(kNB - 1u) ? kNB - 1u : static_cast<uint32_t>(v);
+        return min(static_cast<uint32_t>(v), kNB - 1u);
     }
 };
 
@@ -270,13 +266,19 @@ __device__ void census_clear() {
         const uint32_t c = static_cast<uint32_t>(__popc(w));
         e_wpre()[tid] = wave_incl_scan(c) - c;
         e_cpl()[tid] = w;
-        if (tid == 0) e_sc()[SC_OVF] = 0u;
+        if (tid == 0) {
+            e_sc()[SC_OVF] = 0u;
+            e_sc()[SC_FILED] = 0u;
+        }
     }
+    for (uint32_t b = tid; b < kNB; b += kBlock)
+        e_plan()[b] = (e_plan()[b] & ~PF_REQ) | (bit_of(e_req(), b) ? PF_REQ : 0u);
     TSM_LDS_SYNC();
 }
 
-__device__ __forceinline__ void census_insert(uint32_t key, uint32_t id, uint32_t b) {
+__device__ __noinline__ void census_insert(uint32_t key, uint32_t id, uint32_t b) {
     const uint32_t h = (key * 0x9E3779B1u) >> 21;
+#pragma unroll 1
     for (uint32_t i = 0; i < 64u; i++) {
         const uint32_t s = (h + i) & (kHS - 1u);
         const uint32_t k = atomicCAS(&e_hkey()[s], 0u, key);
@@ -288,6 +290,25 @@ __device__ __forceinline__ void census_insert(uint32_t key, uint32_t id, uint32_
     }
     atomicAnd(&e_cpl()[b >> 5], ~(1u << (b & 31u)));  // no free slot near: the bin stays incomplete
     e_sc()[SC_OVF] = 1u;
+}
+// A pass files the elements it meets in requested bins as composites (in the
+// sort's area, free until census_finish), and the census takes them all at once
+// afterwards: one LDS atomic and a store in the pass's loop instead of a
+// probe.  What does not fit (one bin requested alone, whatever its count) is
+// inserted at once.
+__device__ __forceinline__ void census_file(uint32_t key, uint32_t id, uint32_t b) {
+    const uint32_t at = atomicAdd(&e_sc()[SC_FILED], 1u);
+    if (at < kHS) e_sort()[at] = composite(key, id);
+    else census_insert(key, id, b);
+}
+__device__ __forceinline__ void census_take(const FBins& vb) {
+    TSM_LDS_SYNC();
+    const uint32_t n = min(e_sc()[SC_FILED], kHS);
+    for (uint32_t i = threadIdx.x; i < n; i += kBlock) {
+        const uint64_t c = e_sort()[i];
+        const uint32_t key = ~static_cast<uint32_t>(c >> 32);
+        census_insert(key, static_cast<uint32_t>(c), vb.bin(key_to_float(key)));
+    }
 }
 
 // Turns the census into runs in list order (value descending): key,
@@ -399,25 +420,25 @@ __device__ uint32_t run_steps(float& x, float tau, uint32_t m, float thr, bool* 
             const int g = grid_of(e);
             const uint32_t c = grid_term(tau, e);
             if (c < kBigTerm) {
-                const uint64_t M = static_cast<uint64_t>(ldexpf(x, -g));
+                const uint32_t M = static_cast<uint32_t>(ldexpf(x, -g));  // [2^23, 2^24), less for a subnormal x
                 const uint32_t left = m - done;
                 if (c == 0u) return m;  // every remaining step rounds back to x, and none decides
-                uint64_t n;
+                uint32_t n;
                 if (sub) {
-                    n = M > (1ull << 23) ? (M - (1ull << 23) - 1u) / c : 0u;  // stays above 2^e
+                    n = M > (1u << 23) ? (M - (1u << 23) - 1u) / c : 0u;  // stays above 2^e
                 } else {
-                    n = ((1ull << 24) - M) / c;  // stays at or below 2^(e+1)
+                    n = ((1u << 24) - M) / c;  // stays at or below 2^(e+1)
                     if (K == FK_A) {
-                        const uint64_t mt = static_cast<uint64_t>(ceilf(ldexpf(thr, -g)));
-                        const uint64_t nd = mt > M ? (mt - M - 1u) / c : 0u;  // stays below thr
+                        const uint32_t mt = grid_ceil(thr, g);
+                        const uint32_t nd = mt > M ? (mt - M - 1u) / c : 0u;  // stays below thr
                         n = n < nd ? n : nd;
                     }
                 }
                 if (n > left) n = left;
                 if (n > 0u) {
-                    const uint64_t M2 = sub ? M - n * c : M + n * c;
+                    const uint32_t M2 = sub ? M - n * c : M + n * c;  // at most 2^24
                     x = ldexpf(static_cast<float>(M2), g);
-                    done += static_cast<uint32_t>(n);
+                    done += n;
                     continue;
                 }
             }
@@ -448,7 +469,7 @@ __device__ uint32_t walk_runs(Walk& w, uint32_t r0, uint32_t r1, float T, float 
         if (w.x > 0.0f) {
             const int e = step_binade(w.x, sub);
             const int g = grid_of(e);
-            const uint64_t M = static_cast<uint64_t>(ldexpf(w.x, -g));
+            const uint32_t M = static_cast<uint32_t>(ldexpf(w.x, -g));
             const uint32_t j = i + lane;
             uint32_t mraw = j < r1 ? e_hcnt()[j] : 0u;
             const uint32_t mpre = wave_incl_scan(mraw) - mraw;
@@ -464,27 +485,24 @@ __device__ uint32_t walk_runs(Walk& w, uint32_t r0, uint32_t r1, float T, float 
                 else c = static_cast<uint64_t>(m) * t;
             }
             // past 2^25 units a lane leaves the binade anyway: the clamp keeps
-            // the prefix sums in 32 bits
+            // the prefix sums (and everything below) in 32 bits
             const uint32_t c32 = c > (1ull << 25) ? (1u << 25) : static_cast<uint32_t>(c);
-            const uint64_t incl = wave_incl_scan(c32);
-            const uint64_t excl = incl - c32;
+            const uint32_t incl = wave_incl_scan(c32);
+            const uint32_t excl = incl - c32;
             bool bad = !ok;
             bool restart = false;
             if (sub) {
-                const int64_t end = static_cast<int64_t>(M) - static_cast<int64_t>(incl);
-                bad |= end <= static_cast<int64_t>(1ull << 23);
+                bad |= incl + (1u << 23) >= M;  // the end at or below 2^e
             } else {
-                const uint64_t start = M + excl, end = M + incl;
-                restart = start >= (1ull << 24);
-                bad |= restart || end > (1ull << 24);
-                if (K == FK_A) bad |= end >= static_cast<uint64_t>(ceilf(ldexpf(thr, -g)));
+                restart = M + excl >= (1u << 24);
+                bad |= restart || M + incl > (1u << 24);
+                if (K == FK_A) bad |= M + incl >= grid_ceil(thr, g);
             }
             const uint32_t f = first_lane(wave_ballot(bad));
             const uint32_t fl = f < 64u ? f : 63u;
-            const uint64_t applied = f < 64u ? wave_read64(excl, fl) : wave_read64(incl, 63u);
+            const uint32_t applied = f < 64u ? wave_read(excl, fl) : wave_read(incl, 63u);
             const uint32_t mapplied = f < 64u ? wave_read(mpre, fl) : wave_read(mpre + m, 63u);
-            const uint64_t M2 = sub ? M - applied : M + applied;
-            w.x = ldexpf(static_cast<float>(M2), g);
+            w.x = ldexpf(static_cast<float>(sub ? M - applied : M + applied), g);
             w.pos += mapplied;
             i += f < 64u ? f : 64u;
             if (f == 64u) continue;
@@ -546,8 +564,8 @@ __device__ uint32_t walk_bins(Walk& w, uint32_t bend, uint32_t nruns, float T, f
             // kBL bins per lane: lane l takes bins w.b + kBL*l .. + kBL-1
             const int e = step_binade(w.x, sub);
             const int g = grid_of(e);
-            const uint64_t M = static_cast<uint64_t>(ldexpf(w.x, -g));
-            const uint64_t mthr = K == FK_A ? static_cast<uint64_t>(ceilf(ldexpf(thr, -g))) : 0u;
+            const uint32_t M = static_cast<uint32_t>(ldexpf(w.x, -g));
+            const uint32_t mthr = K == FK_A ? grid_ceil(thr, g) : 0u;
             const uint32_t bl = w.b + kBL * lane;
             uint32_t nj[kBL], cj[kBL];
             bool okj[kBL];
@@ -557,7 +575,7 @@ __device__ uint32_t walk_bins(Walk& w, uint32_t bend, uint32_t nruns, float T, f
                 const uint32_t b = bl + j;
                 uint32_t n = 0;
                 bool ok = b < bend;  // past bend: the end marker
-                uint64_t c = 0;
+                uint32_t c = 0;
                 if (ok) {
                     n = e_cnt()[b];
                     if (n) {
@@ -574,14 +592,14 @@ __device__ uint32_t walk_bins(Walk& w, uint32_t bend, uint32_t nruns, float T, f
                              (kB == 0 ? !tie_bit(slot, b) : !bad_bit(slot, b));
                         if (ok) {
                             const bool tie = kB != 0 && tie_bit(slot, b);
-                            c = static_cast<uint64_t>(e_sum(slot)[b]) + (kB == 2 && tie ? 1u : 0u);
+                            c = min(e_sum(slot)[b], 1u << 25) + (kB == 2 && tie ? 1u : 0u);
                             if (tie) tmask |= 1u << j;
                         }
                     }
                 }
                 // past 2^25 units a bin leaves the binade anyway: the clamps keep
                 // the prefix sums in 32 bits
-                cj[j] = c > (1ull << 25) ? (1u << 25) : static_cast<uint32_t>(c);
+                cj[j] = min(c, 1u << 25);
                 nj[j] = n;
                 okj[j] = ok;
                 ln += n;
@@ -591,22 +609,21 @@ __device__ uint32_t walk_bins(Walk& w, uint32_t bend, uint32_t nruns, float T, f
             const uint32_t cpre = wave_incl_scan(lc) - lc;
             uint32_t jb = kBL;  // the lane's first bin the sums cannot take
             bool restart = false;
-            uint64_t pre = cpre;
+            uint32_t pre = cpre;  // at most 64 * 2^25, and four bins more: 32 bits
             uint32_t np = npre;
-            uint64_t pre_at = 0;
+            uint32_t pre_at = 0;
             uint32_t np_at = 0;
 #pragma unroll
             for (uint32_t j = 0; j < kBL; j++) {
-                const uint64_t start = sub ? M - pre : M + pre;
+                const uint32_t start = sub ? M - pre : M + pre;
                 bool bad = !okj[j];
                 bool rs = false;
                 if (sub) {
-                    const int64_t end = static_cast<int64_t>(M) - static_cast<int64_t>(pre + cj[j]);
-                    bad |= nj[j] > 0u && end <= static_cast<int64_t>(1ull << 23);
+                    bad |= nj[j] > 0u && pre + cj[j] + (1u << 23) >= M;  // the end at or below 2^e
                 } else {
-                    const uint64_t end = M + pre + cj[j];
-                    rs = start >= (1ull << 24);
-                    bad |= rs || end > (1ull << 24);
+                    const uint32_t end = start + cj[j];
+                    rs = start >= (1u << 24);
+                    bad |= rs || end > (1u << 24);
                     if (K == FK_A) bad |= nj[j] > 0u && end >= mthr;
                 }
                 if (jb == kBL) {
@@ -634,13 +651,13 @@ __device__ uint32_t walk_bins(Walk& w, uint32_t bend, uint32_t nruns, float T, f
             // lanes after f recorded bin starts past the stop; the next step
             // writes them again from the right value
             if (f == 64u) {
-                const uint64_t applied = wave_read64(pre, 63u);  // cpre + lc of the last lane
+                const uint32_t applied = wave_read(pre, 63u);  // cpre + lc of the last lane
                 w.x = ldexpf(static_cast<float>(sub ? M - applied : M + applied), g);
                 w.pos += wave_read(np, 63u);
                 w.b += kBL * 64u;
                 continue;
             }
-            const uint64_t applied = wave_read64(pre_at, f);
+            const uint32_t applied = wave_read(pre_at, f);
             w.x = ldexpf(static_cast<float>(sub ? M - applied : M + applied), g);
             w.pos += wave_read(np_at, f);
             w.b = wave_read(bl + jb, f);
@@ -675,15 +692,18 @@ __device__ __forceinline__ bool fold_needs(int k, uint32_t b, bool exact) {
 }
 
 // ---- passes ----------------------------------------------------------------
-// tau's grid units for the sums of slot `slot` (binade g); a step that
-// cannot be summed, or a sum that could pass 2^32 over the bin's n
-// candidates, marks the bin's sum invalid.
+// tau's grid units for the sums of slot `slot` (the grid of binade g, g >=
+// -126); a step that cannot be summed, or a sum that could pass 2^32 over the
+// bin's n candidates, marks the bin's sum invalid.  The same units as
+// grid_term, by rounding tau / grid to the nearest integer: a tie is where that
+// moved it by a half.
 __device__ __forceinline__ void add_term(uint32_t slot, uint32_t b, float tau, int g, uint32_t n) {
-    uint32_t fl = 0;
-    uint32_t t = grid_term(tau, g, &fl);
-    const bool tie = t == kTieTerm;
-    if (tie) t = fl;  // the lower bound of the step; the tie bit says it may be one more
-    const bool bad = t == kBigTerm || static_cast<uint64_t>(t) * n >= (1ull << 32);
+    const float v = ldexpf(tau, 23 - g);
+    const float r = rintf(v), d = v - r;
+    const bool tie = fabsf(d) == 0.5f;
+    // a tie takes its lower end; the tie bit says it may be one more
+    const uint32_t t = static_cast<uint32_t>(tie ? floorf(v) : r);
+    const bool bad = !(v < 16777216.0f) || (n > 255u && static_cast<uint64_t>(t) * n >= (1ull << 32));
     atomicAdd(&e_sum(slot)[b], bad ? 0u : t);
     if (bad || tie) {
         const uint32_t i = slot * kNB + b;
@@ -691,6 +711,16 @@ __device__ __forceinline__ void add_term(uint32_t slot, uint32_t b, float tau, i
         const uint32_t old = atomicOr(&e_tie()[i >> 5], bit);
         if (bad || (old & bit)) atomicOr(&e_tieb()[i >> 5], bit);
     }
+}
+
+// a / b rounded to f32, for f32 a and b with inv = 1 / b in f64: the product's
+// relative error is below 2^-51, and no quotient of two f32 values lies within
+// 2^-49 of the middle between two f32 values (its distance from one is a
+// nonzero multiple of 2^-24 / b in units of the middle's last place), so it
+// rounds as the quotient does.  (A subnormal quotient may round otherwise: exp
+// of it is 1 either way.)  A third of the instructions of the f32 division.
+__device__ __forceinline__ float quotient(float a, double inv) {
+    return static_cast<float>(static_cast<double>(a) * inv);
 }
 
 enum : int { EP_HIST = 0, EP_SR = 1, EP_A = 2, EP_CENSUS = 3, EP_SUB = 4 };
@@ -704,13 +734,22 @@ enum : int { EP_HIST = 0, EP_SR = 1, EP_A = 2, EP_CENSUS = 3, EP_SUB = 4 };
 //   EP_CENSUS  the census alone;
 //   EP_SUB     the crowded coarse bins' sub-histograms (kSub bins each, in
 //              e_hkey, which holds no census yet).
-// The row is read as in row_pass (16-byte blocks, the next tile in flight);
-// each element takes one predicate and one branch into the mode's work.
+// The row is read by row_blocks, four elements at a time.
 template <int kMode>
 __device__ __noinline__ void eng_pass(Fin& f_in, const Filt& q_in, const FBins& vb_in, float T) {
     const Fin f = f_in;  // a private copy: its fields stay in registers across LDS atomics
-    const Filt q = q_in;
-    const FBins vb = vb_in;
+    // the same for every lane: in scalar registers
+    Filt q = q_in;
+    q.use_cut = wave_uniform(q.use_cut ? 1u : 0u) != 0u;
+    q.use_max = wave_uniform(q.use_max ? 1u : 0u) != 0u;
+    q.need_allowed = wave_uniform(q.need_allowed ? 1u : 0u) != 0u;
+    q.use_minp = wave_uniform(q.use_minp ? 1u : 0u) != 0u;
+    FBins vb = vb_in;
+    vb.vb.y0 = wave_uniform_f(vb.vb.y0);
+    vb.vb.mul = wave_uniform_f(vb.vb.mul);
+    vb.scale = wave_uniform_f(vb.scale);
+#pragma unroll
+    for (uint32_t s = 0; s < kCrowd; s++) vb.cr[s] = wave_uniform(vb.cr[s]);
     const uint32_t tid = threadIdx.x;
     if (kMode == EP_HIST) {
         for (uint32_t i = tid; i < kNB; i += kBlock) {
@@ -732,142 +771,113 @@ __device__ __noinline__ void eng_pass(Fin& f_in, const Filt& q_in, const FBins& 
         }
     }
     TSM_LDS_SYNC();
-    const float t = f.m.t;
+    const float t = wave_uniform_f(f.m.t);
     const float y0 = vb.vb.y0;
     const float l2t = 1.4426950408889634f / t;
+    const double invt = 1.0 / static_cast<double>(t), invT = 1.0 / static_cast<double>(T);
     const uint64_t* tab = e_exptab();
-    uint32_t kmin = 0xFFFFFFFFu;
+    float ymin = INFINITY;
     bool nan = false;
+    const TSM_GLOBAL_AS uint32_t* mrow = global_as(wave_uniform_p(f.mrow));
+    // without a cut every id is a candidate, NaNs too: they fail a compare with
+    // the cut, as they should with one, and are taken up by `more`
+    const bool nocut = !q.use_cut, more = nocut || q.use_max || q.need_allowed || q.use_minp;
+    const float cut = nocut ? -INFINITY : wave_uniform_f(q.cut);
 
-    const uint32_t n = f.n;
-    const bool penal = f.m.penal;
-    const TSM_GLOBAL_AS float* rowp = global_as(f.rowp);
-    const TSM_GLOBAL_AS uint32_t* mrow = global_as(f.mrow);
-    const uint32_t head = static_cast<uint32_t>((reinterpret_cast<uintptr_t>(f.rowp) >> 2) & 3u);
-    const TSM_GLOBAL_AS float* base = rowp - head;  // 16-byte aligned
-    const uint32_t span = head + n, nblk = (span + 3u) / 4u, full = span / 4u;
-    constexpr uint32_t kTB = kReTile / 4u;
-    constexpr uint32_t kPer = kTB / kBlock;
-    const TSM_GLOBAL_AS uint32_t* hist = global_as(f.hist);
-    const uint32_t hc = min(f.hlen, TSM_MAX_HISTORY);
-    auto load_blk = [&](uint32_t j) -> float4 {
-        if (j < full && (j > 0u || head == 0u)) return load4(base + 4u * j);
-        float4 r = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (j < nblk) {
-            const uint32_t i0 = 4u * j;
-            if (i0 >= head && i0 < span) r.x = rowp[i0 - head];
-            if (i0 + 1u >= head && i0 + 1u < span) r.y = rowp[i0 + 1u - head];
-            if (i0 + 2u >= head && i0 + 2u < span) r.z = rowp[i0 + 2u - head];
-            if (i0 + 3u >= head && i0 + 3u < span) r.w = rowp[i0 + 3u - head];
-        }
-        return r;
-    };
-    float4 cur[kPer], nxt[kPer];
+    row_blocks(f, [&](uint32_t id0, uint32_t in, const float (&)[4], const float (&y)[4]) __attribute__((always_inline)) {
+        bool keep[4];
 #pragma unroll
-    for (uint32_t k = 0; k < kPer; k++) cur[k] = load_blk(tid + k * kBlock);
-    const uint32_t ntiles = (nblk + kTB - 1u) / kTB;
-    for (uint32_t tl = 0; tl < ntiles; tl++) {
-        if (tl + 1u < ntiles) {
-#pragma unroll
-            for (uint32_t k = 0; k < kPer; k++) nxt[k] = load_blk((tl + 1u) * kTB + tid + k * kBlock);
-        }
-        const uint32_t tb = tl * kReTile;
-        if (penal) {
-            TSM_LDS_SYNC();
-            for (uint32_t i = tid; i < kReTile / 2; i += kBlock) f.cnt()[i] = 0;
-            TSM_LDS_SYNC();
-            for (uint32_t h = tid; h < hc; h += kBlock) {
-                const uint32_t li = hist[h] + head - tb;
-                if (li < kReTile && hist[h] < n) atomicAdd(&f.cnt()[li >> 1], 1u << ((li & 1u) << 4));
-            }
-            TSM_LDS_SYNC();
-        }
-#pragma unroll
-        for (uint32_t k = 0; k < kPer; k++) {
-            const uint32_t j = tl * kTB + tid + k * kBlock;
-            const float xv[4] = {cur[k].x, cur[k].y, cur[k].z, cur[k].w};
+        for (uint32_t e = 0; e < 4u; e++) keep[e] = ((in >> e) & 1u) && y[e] >= cut;
+        if (more) {
 #pragma unroll
             for (uint32_t e = 0; e < 4u; e++) {
-                const uint32_t i = 4u * j + e;
-                const uint32_t id = i - head;
-                bool keep = j < nblk && i >= head && i < span;
-                float y = xv[e];
-                if (penal) {
-                    const uint32_t li = (i - tb) & (kReTile - 1u);
-                    const uint32_t c = (f.cnt()[li >> 1] >> ((li & 1u) << 4)) & 0xFFFFu;
-                    if (c) y = penalize(y, c, f.m, f.P);
+                const uint32_t id = id0 + e;
+                bool k = keep[e] || (nocut && ((in >> e) & 1u));
+                if (q.use_max) k = k && composite(total_key(y[e]), id) <= q.max_comp;
+                if (q.need_allowed && k) k = (mrow[id >> 5] >> (id & 31u)) & 1u;
+                if (q.use_minp && k) {
+                    k = !(y[e] < q.minp_lo);
+                    if (k && !(y[e] >= q.minp_hi))
+                        k = glibc_expf_lds(quotient(y[e] - q.y0, invt), tab) >= q.minp;
                 }
-                if (q.use_cut) keep = keep && y >= q.cut;
-                if (q.use_max) keep = keep && composite(total_key(y), id) <= q.max_comp;
-                if (q.need_allowed && keep) keep = (mrow[id >> 5] >> (id & 31u)) & 1u;
-                if (q.use_minp && keep) {
-                    keep = !(y < q.minp_lo);
-                    if (keep && !(y >= q.minp_hi)) keep = glibc_expf_lds((y - q.y0) / t, tab) >= q.minp;
-                }
-                if (kMode == EP_SUB) {
-                    if (keep && y == y) {
-                        const uint32_t c = vb.vb.bin(y);
+                keep[e] = k;
+            }
+        }
+        if (kMode == EP_SUB) {
 #pragma unroll
-                        for (uint32_t s = 0; s < kCrowd; s++) {
-                            if (c != vb.cr[s]) continue;
-                            const float x = vb.frac(y, c) * static_cast<float>(kSub);
-                            const uint32_t j = x < static_cast<float>(kSub - 1u) ? static_cast<uint32_t>(x) : kSub - 1u;
-                            atomicAdd(&e_hkey()[s * kSub + j], 1u);
-                        }
-                    }
-                    continue;
+            for (uint32_t e = 0; e < 4u; e++) {
+                if (!(keep[e] && y[e] == y[e])) continue;
+                const uint32_t c = vb.vb.bin(y[e]);
+#pragma unroll
+                for (uint32_t s = 0; s < kCrowd; s++) {
+                    if (c != vb.cr[s]) continue;
+                    const float x = vb.frac(y[e], c) * static_cast<float>(kSub);
+                    const uint32_t j = x < static_cast<float>(kSub - 1u) ? static_cast<uint32_t>(x) : kSub - 1u;
+                    atomicAdd(&e_hkey()[s * kSub + j], 1u);
                 }
-                const uint32_t b = vb.bin(y);
-                if (kMode == EP_HIST) {
-                    const bool isnan = y != y;
-                    nan |= keep && isnan;
-                    keep = keep && !isnan;
-                    const double m = static_cast<double>(__builtin_amdgcn_exp2f((y - y0) * l2t));
-                    const uint32_t kk = total_key(y);
-                    kmin = keep && kk < kmin ? kk : kmin;
-                    if (keep) {
-                        atomicAdd(&e_cnt()[b], 1u);
-                        atomicAdd(&e_mass()[b], m);
-                    }
-                } else {
-                    if (kMode != EP_CENSUS) {
-                        const uint32_t pw = e_plan()[b];
-                        const uint32_t nb = e_cnt()[b];
-                        const float p = glibc_expf_lds((y - y0) / t, tab);
-                        if (kMode == EP_SR) {
-                            const int gs = static_cast<int>(pw & 0xFFu) - 128;
-                            const int gr = static_cast<int>((pw >> 8) & 0xFFu) - 128;
-                            const bool ds = keep && !(pw & PF_MUST_S);
-                            const bool dr = keep && (pw & PF_R) && !(pw & PF_MUST_R);
-                            if (ds) {
-                                add_term(SL_S0, b, p, gs, nb);
-                                if (pw & PF_TWO_S) add_term(SL_S1, b, p, gs + 1, nb);
-                            }
-                            if (dr) {
-                                add_term(SL_R0, b, p, gr, nb);
-                                if (pw & PF_TWO_R) add_term(SL_R1, b, p, gr + 1, nb);
-                            }
-                        } else {
-                            const float qv = p / T;
-                            const int ga = static_cast<int>((pw >> 16) & 0xFFu) - 128;
-                            if (keep && !(pw & PF_MUST_A)) {
-                                add_term(SL_S0, b, qv, ga, nb);
-                                if (pw & PF_TWO_A) add_term(SL_S1, b, qv, ga + 1, nb);
-                            }
-                        }
-                    }
-                    if (keep && bit_of(e_req(), b)) census_insert(total_key(y), id, b);
+            }
+            return;
+        }
+        // the four elements' lookups first, then their updates: the LDS reads
+        // of one element do not wait behind another's atomics
+        uint32_t b[4];
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; e++) b[e] = vb.bin(y[e]);
+        if (kMode == EP_HIST) {
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; e++) {
+                const bool isnan = y[e] != y[e];
+                nan |= keep[e] && isnan;
+                if (keep[e] && !isnan) {
+                    const double m = static_cast<double>(__builtin_amdgcn_exp2f((y[e] - y0) * l2t));
+                    ymin = fminf(ymin, y[e]);
+                    atomicAdd(&e_cnt()[b[e]], 1u);
+                    atomicAdd(&e_mass()[b[e]], m);
+                }
+            }
+            return;
+        }
+        uint32_t pw[4], nb[4];
+        float p[4];
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; e++) {
+            pw[e] = e_plan()[b[e]];
+            if (kMode != EP_CENSUS) {
+                nb[e] = e_cnt()[b[e]];
+                p[e] = glibc_expf_lds(quotient(y[e] - y0, invt), tab);
+                if (kMode == EP_A) p[e] = quotient(p[e], invT);
+            }
+        }
+        if (kMode == EP_SR || kMode == EP_A) {
+            constexpr uint32_t sh = kMode == EP_SR ? 0u : 16u;
+            constexpr uint32_t must = kMode == EP_SR ? PF_MUST_S : PF_MUST_A, two = kMode == EP_SR ? PF_TWO_S : PF_TWO_A;
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; e++) {
+                const int g = static_cast<int>((pw[e] >> sh) & 0xFFu) - 128;
+                if (keep[e] && !(pw[e] & must)) {
+                    add_term(SL_S0, b[e], p[e], g, nb[e]);
+                    if (pw[e] & two) add_term(SL_S1, b[e], p[e], g + 1, nb[e]);
                 }
             }
         }
-        if (tl + 1u < ntiles) {
+        if (kMode == EP_SR) {
 #pragma unroll
-            for (uint32_t k = 0; k < kPer; k++) cur[k] = nxt[k];
+            for (uint32_t e = 0; e < 4u; e++) {
+                const int g = static_cast<int>((pw[e] >> 8) & 0xFFu) - 128;
+                if (keep[e] && (pw[e] & PF_R) && !(pw[e] & PF_MUST_R)) {
+                    add_term(SL_R0, b[e], p[e], g, nb[e]);
+                    if (pw[e] & PF_TWO_R) add_term(SL_R1, b[e], p[e], g + 1, nb[e]);
+                }
+            }
         }
-    }
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; e++)
+            if (keep[e] && (pw[e] & PF_REQ)) census_file(total_key(y[e]), id0 + e, b[e]);
+    });
+    if (kMode == EP_SR || kMode == EP_A || kMode == EP_CENSUS) census_take(vb);
     if (kMode == EP_HIST) {
         TSM_LDS_SYNC();
-        kmin = wave_min(kmin);
+        const uint32_t kmin = wave_min(ymin == INFINITY ? 0xFFFFFFFFu : total_key(ymin));
         if (lane_id() == 0 && kmin != 0xFFFFFFFFu) atomicMin(&e_sc()[SC_CMIN], kmin);
         if (nan) e_sc()[SC_NAN] = 1u;
     }
@@ -883,6 +893,8 @@ constexpr double kPlanEps = 1e-4;
 // The same for predicting where a fold will step value by value (census
 // requests): tighter, since a miss costs a census round, not a wrong result.
 constexpr double kPredEps = 2e-5;
+// ... and, of the total, for the draw's value.
+constexpr double kDrawSlack = 1e-5;
 
 __device__ __forceinline__ void plan_range(double lo, double hi, bool sub, uint32_t shift, uint32_t two,
                                            uint32_t must, uint32_t* pw) {
@@ -896,9 +908,49 @@ __device__ __forceinline__ void plan_range(double lo, double hi, bool sub, uint3
     if (e_hi > e_lo) *pw |= two;
 }
 
+// What a fold moves by over a bin of n candidates of approximate mass m when
+// its value there is about x: each step rounds to the grid of x's binade, which
+// drops or doubles terms not far above the grid (f32 folds of 150,000 terms end
+// up to 2e-4 off the sum because of it).  A bin is narrow: its terms are taken
+// as spread evenly over a stretch `wide` of their mean wide, which holds at most
+// one step of the rounding.
+__device__ __forceinline__ double fold_mass(double m, uint32_t n, double x, bool sub, double wide) {
+    if (!n || !(x > 0.0)) return m;
+    const double unit = ldexp(1.0, grid_of(step_binade(static_cast<float>(x), sub)));
+    const double v = m / (static_cast<double>(n) * unit);
+    if (!(v < 64.0)) return m;
+    const double k = floor(v), up = (v * (1.0 + 0.5 * wide) - (k + 0.5)) / (v * wide);
+    return static_cast<double>(n) * (k + fmin(fmax(up, 0.0), 1.0)) * unit;
+}
+// This thread's two bins' masses and the cumulative ones before them, as total's
+// fold and as the draw's (from r = u * kept) see them.
+struct FoldView {
+    double S[2], ms[2], R[2], mr[2];  // cumulative, own
+    double tot, kept;                 // total's fold; about its part up to top_p
+};
+// `wide`: a coarse bin's width, relative to its terms.
+__device__ FoldView fold_view(Fin& f, const double (&m)[2], const uint32_t (&c)[2], float u, bool draw, bool topp,
+                              double wide) {
+    FoldView w;
+    double t0;
+    const double P0 = block_excl_scan_f64(m[0] + m[1], f.miscd() + 8, &t0);
+    w.ms[0] = fold_mass(m[0], c[0], P0, false, wide);
+    w.ms[1] = fold_mass(m[1], c[1], P0 + m[0], false, wide);
+    w.S[0] = block_excl_scan_f64(w.ms[0] + w.ms[1], f.miscd() + 8, &w.tot);
+    w.S[1] = w.S[0] + w.ms[0];
+    w.kept = topp ? fmin(static_cast<double>(f.P.top_p), 1.0) * w.tot : w.tot;
+    const double r0 = static_cast<double>(u) * w.kept;
+    w.mr[0] = draw ? fold_mass(m[0], c[0], r0 - w.S[0], true, wide) : w.ms[0];
+    w.mr[1] = draw ? fold_mass(m[1], c[1], r0 - w.S[1], true, wide) : w.ms[1];
+    double rt = 0.0;
+    w.R[0] = draw ? block_excl_scan_f64(w.mr[0] + w.mr[1], f.miscd() + 8, &rt) : w.S[0];
+    w.R[1] = w.R[0] + w.mr[0];
+    return w;
+}
+
 // Plans of total and the draw from the approximate masses, with the bins each
 // is expected to step through.  Two bins per thread.
-__device__ void plan_sr(Fin& f, float u, bool draw, bool topp) {
+__device__ void plan_sr(Fin& f, float u, bool draw, bool topp, double wide) {
     const uint32_t tid = threadIdx.x;
     const uint32_t b0 = 2 * tid;
     for (uint32_t i = tid; i < 3u * kNB / 32u; i += kBlock) e_xreq(0)[i] = 0u;
@@ -906,18 +958,16 @@ __device__ void plan_sr(Fin& f, float u, bool draw, bool topp) {
         e_sc()[SC_KLO] = 0xFFFFFFFFu;
         e_sc()[SC_KHI] = 0u;
     }
-    const double m0 = e_mass()[b0], m1 = e_mass()[b0 + 1];
-    const uint32_t c0 = e_cnt()[b0], c1 = e_cnt()[b0 + 1];
-    double tot;
-    const double P0 = block_excl_scan_f64(m0 + m1, f.miscd() + 8, &tot);  // barriers order the clears above
-    const double Pb[2] = {P0, P0 + m0}, mb[2] = {m0, m1};
-    const uint32_t cb[2] = {c0, c1};
+    const double mb[2] = {e_mass()[b0], e_mass()[b0 + 1]};
+    const uint32_t cb[2] = {e_cnt()[b0], e_cnt()[b0 + 1]};
+    const FoldView w = fold_view(f, mb, cb, u, draw, topp, wide);  // barriers order the clears above
+    const double tot = w.tot;
     const double tp = static_cast<double>(f.P.top_p);
     const double eps2 = kPredEps;
     if (topp) {
 #pragma unroll
         for (int k = 0; k < 2; k++)
-            if (cb[k] && (Pb[k] + mb[k]) / tot >= tp - eps2 && Pb[k] / tot <= tp + eps2) {
+            if (cb[k] && (w.S[k] + w.ms[k]) / tot >= tp - eps2 && w.S[k] / tot <= tp + eps2) {
                 atomicMin(&e_sc()[SC_KLO], b0 + k);
                 atomicMax(&e_sc()[SC_KHI], b0 + k);
             }
@@ -926,8 +976,8 @@ __device__ void plan_sr(Fin& f, float u, bool draw, bool topp) {
     const uint32_t klo = e_sc()[SC_KLO], khi = e_sc()[SC_KHI];
 #pragma unroll
     for (int k = 0; k < 2; k++) {  // the kept mass's bounds: cumulative masses at the region's ends
-        if (topp && klo != 0xFFFFFFFFu && b0 + k == klo) e_scd()[0] = Pb[k];
-        if (topp && klo != 0xFFFFFFFFu && b0 + k == khi) e_scd()[1] = Pb[k] + mb[k];
+        if (topp && klo != 0xFFFFFFFFu && b0 + k == klo) e_scd()[0] = w.S[k];
+        if (topp && klo != 0xFFFFFFFFu && b0 + k == khi) e_scd()[1] = w.S[k] + w.ms[k];
     }
     TSM_LDS_SYNC();
     double M_lo = tot, M_hi = tot;
@@ -938,10 +988,11 @@ __device__ void plan_sr(Fin& f, float u, bool draw, bool topp) {
     M_lo *= 1.0 - kPredEps;
     M_hi *= 1.0 + kPredEps;
     const double du = static_cast<double>(u);
-    // r = u * mass - (total's fold so far) carries the drift of both f32
-    // folds over the whole row (total's own reaches ~1e-5 of it): an absolute
-    // margin of 1e-4 of the total
-    const double slack = 1e-4 * tot;
+    // r carries what the estimates leave of the drift of both f32 folds over
+    // the whole row: an absolute margin.  A draw that ends deep in the tail
+    // stays inside the margin for long, and every bin there is stepped value by
+    // value.
+    const double slack = kDrawSlack * tot;
 #pragma unroll
     for (int k = 0; k < 2; k++) {
         const uint32_t b = b0 + k;
@@ -950,23 +1001,23 @@ __device__ void plan_sr(Fin& f, float u, bool draw, bool topp) {
             continue;
         }
         uint32_t pw = 0;
-        // total: the fold value at the bin's start is about Pb
-        const double slo = Pb[k] * (1.0 - kPlanEps), shi = Pb[k] * (1.0 + kPlanEps);
+        // total: the fold value at the bin's start is about S
+        const double slo = w.S[k] * (1.0 - kPlanEps), shi = w.S[k] * (1.0 + kPlanEps);
         plan_range(slo, shi, false, 0u, PF_TWO_S, PF_MUST_S, &pw);
-        if ((pw & PF_MUST_S) || binade_of(static_cast<float>((Pb[k] + mb[k]) * (1.0 + kPlanEps))) !=
+        if ((pw & PF_MUST_S) || binade_of(static_cast<float>((w.S[k] + w.ms[k]) * (1.0 + kPlanEps))) !=
                                      binade_of(static_cast<float>(slo)))
             set_bit(e_xreq(FK_S), b);
         if (draw) {
-            // the draw: r at the bin's start is about u * M - Pb
-            const double rlo = du * M_lo - Pb[k] * (1.0 + kPredEps) - slack,
-                         rhi = du * M_hi - Pb[k] * (1.0 - kPredEps) + slack;
+            // the draw: r at the bin's start is about u * M - R
+            const double rlo = du * M_lo - w.R[k] * (1.0 + kPredEps) - slack,
+                         rhi = du * M_hi - w.R[k] * (1.0 - kPredEps) + slack;
             if (rhi > 0.0) {
                 pw |= PF_R;
                 plan_range(rlo, rhi, true, 8u, PF_TWO_R, PF_MUST_R, &pw);
                 // r may leave its binade (or reach zero) in this bin when the
                 // lowest end value and the highest start value lie in
                 // different binades
-                const double elo = rlo - mb[k] * (1.0 + kPredEps);
+                const double elo = rlo - w.mr[k] * (1.0 + kPredEps);
                 if ((pw & PF_MUST_R) || !(elo > 0.0) ||
                     binade_of(static_cast<float>(elo)) != step_binade(static_cast<float>(rhi), true))
                     set_bit(e_xreq(FK_R), b);
@@ -1047,17 +1098,28 @@ __device__ uint2 trim_bins(uint32_t& w, uint32_t cap_cnt, uint32_t cap_bins, boo
 // left, those of the folds still to come (acc's when acc_next, the draw's
 // when draw).  Within kReqCnt candidates and kReqMax bins, lowest bins first.
 __device__ void request_round(int K, uint32_t from, bool draw, bool acc_next, bool exact, bool whole = false) {
+    // every thread judges its bins, a wave's 64 by ballots; wave 0 then trims
+    // the two bitmaps, a word a lane (e_req: this fold's, e_tmpb: the others')
     const uint32_t tid = threadIdx.x;
-    if (tid < kWave) {
-        uint32_t cur = 0, later = 0;
-        for (uint32_t i = 0; i < 32u; i++) {
-            const uint32_t b = 32u * tid + i;
-            if (!e_cnt()[b]) continue;
-            if (b == from || (b > from && fold_needs(K, b, exact))) cur |= 1u << i;
-            else if ((whole && fold_needs(K, b, exact)) || (K == FK_S && ((acc_next && bit_of(e_xreq(FK_A), b)) || (draw && fold_needs(FK_R, b, false)))) ||
-                     (K == FK_A && draw && fold_needs(FK_R, b, false)))
-                later |= 1u << i;
+    for (uint32_t b = tid; b < kNB; b += kBlock) {
+        bool now = false, after = false;
+        if (e_cnt()[b]) {
+            const bool needs = fold_needs(K, b, exact);
+            now = b == from || (b > from && needs);
+            after = !now && ((whole && needs) ||
+                             (K == FK_S && ((acc_next && bit_of(e_xreq(FK_A), b)) || (draw && fold_needs(FK_R, b, false)))) ||
+                             (K == FK_A && draw && fold_needs(FK_R, b, false)));
         }
+        const uint64_t bn = wave_ballot(now), ba = wave_ballot(after);
+        if (lane_id() < 2u) {
+            const uint32_t w = (b & ~(kWave - 1u)) / 32u + lane_id();
+            e_req()[w] = static_cast<uint32_t>(lane_id() ? bn >> 32 : bn);
+            e_tmpb()[w] = static_cast<uint32_t>(lane_id() ? ba >> 32 : ba);
+        }
+    }
+    TSM_LDS_SYNC();
+    if (tid < kWave) {
+        uint32_t cur = e_req()[tid], later = e_tmpb()[tid];
         const uint2 used = trim_bins(cur, kReqCnt, kReqMax, true);
         const uint32_t room_c = used.x < kReqCnt ? kReqCnt - used.x : 0u;
         const uint32_t room_b = used.y < kReqMax ? kReqMax - used.y : 0u;
@@ -1242,28 +1304,25 @@ __device__ __forceinline__ bool locate(uint32_t lb, uint32_t pos, uint32_t nruns
 constexpr uint32_t kHot = 32;  // weight factor of coarse bins where a fold steps value by value
 constexpr uint32_t kFineCap = 1024;  // candidates a fine bin's share of the weight may hold
 
-// Does a coarse bin of approximate mass m after cumulative mass P (of tot)
-// hold a predicted event: total crossing a power of two, acc = total / tot
-// crossing one, top-p's decision, or r = u * mass - P crossing one or
-// reaching zero?  The margins cover the gap between these estimates and the
+// Does this thread's coarse bin k hold a predicted event: total crossing a
+// power of two, acc = total / tot crossing one, top-p's decision, or the
+// draw's r crossing one or reaching zero?  The margins cover the gap between these estimates and the
 // f32 folds.
-__device__ __forceinline__ bool coarse_hot(double P, double m, double tot, float u, bool topp, bool draw,
-                                           float top_p) {
-    if (m <= 0.0) return false;
-    const double lo = P * (1.0 - kPlanEps), hi = (P + m) * (1.0 + kPlanEps);
+__device__ __forceinline__ bool coarse_hot(const FoldView& w, int k, float u, bool topp, bool draw, float top_p) {
+    if (w.ms[k] <= 0.0 && w.mr[k] <= 0.0) return false;
+    const double lo = w.S[k] * (1.0 - kPlanEps), hi = (w.S[k] + w.ms[k]) * (1.0 + kPlanEps);
     if (!(lo > 0.0) || binade_of(static_cast<float>(lo)) != binade_of(static_cast<float>(hi))) return true;
     if (topp) {
         // acc stops at top_p: a bin that starts past it is never walked by acc
-        const double tp = static_cast<double>(top_p) * tot;
+        const double tp = static_cast<double>(top_p) * w.tot;
         if (lo <= tp * (1.0 + kPlanEps)) {
-            if (binade_of(static_cast<float>(lo / tot)) != binade_of(static_cast<float>(hi / tot))) return true;
+            if (binade_of(static_cast<float>(lo / w.tot)) != binade_of(static_cast<float>(hi / w.tot))) return true;
             if (tp <= hi) return true;
         }
     }
     if (draw) {
-        const double M = topp ? static_cast<double>(top_p) * tot : tot;
-        const double rhi = static_cast<double>(u) * M * (1.0 + kPlanEps) - lo;
-        const double rlo = static_cast<double>(u) * M * (1.0 - kPlanEps) - hi;
+        const double r0 = static_cast<double>(u) * w.kept, eps = kPlanEps * r0;
+        const double rhi = r0 - w.R[k] + eps, rlo = r0 - (w.R[k] + w.mr[k]) - eps;
         if (rhi > 0.0 && (!(rlo > 0.0) || binade_of(static_cast<float>(rlo)) != binade_of(static_cast<float>(rhi))))
             return true;
     }
@@ -1297,7 +1356,7 @@ __device__ __noinline__ bool crowd_layout(Fin& f, const Filt& q, FBins& vb, uint
     for (uint32_t k = 0; k < 2u; k++) {
         const uint32_t c = 2u * tid + k;
         if ((k == 0u ? cnt0 : cnt1) <= kReqCnt / 4u) continue;  // too few to crowd a fine bin
-        const uint32_t l0 = e_lay()[c], l1 = c + 1u < kNB ? e_lay()[c + 1u] : l0 + (kNB - 1u);
+        const uint32_t l0 = e_lay()[c], l1 = e_lay()[c + 1u];
         const uint32_t f0 = min(static_cast<uint32_t>(static_cast<float>(l0) * vb.scale), kNB - 1u);
         const uint32_t f1 = min(static_cast<uint32_t>(static_cast<float>(l1) * vb.scale), kNB - 1u);
         bool crowded = false;
@@ -1444,10 +1503,11 @@ __device__ __noinline__ BigOut big_nucleus(Fin& f_in, const Filt& q_in, float y0
             // (a binade crossing of total, acc or r, top-p's decision, the
             // draw's end), so that those stretches are censused in small bins
             const double m0 = e_mass()[2 * tid], m1 = e_mass()[2 * tid + 1];
-            double mtot;
-            const double P0 = block_excl_scan_f64(m0 + m1, f.miscd() + 8, &mtot);
-            const bool h0 = coarse_hot(P0, m0, mtot, u, topp, draw, f.P.top_p);
-            const bool h1 = coarse_hot(P0 + m0, m1, mtot, u, topp, draw, f.P.top_p);
+            const double wide = 1.0 / (static_cast<double>(vb.vb.mul) * t);
+            const double mm[2] = {m0, m1};
+            const uint32_t cc[2] = {c0, c1};
+            const FoldView w = fold_view(f, mm, cc, u, draw, topp, wide);
+            const bool h0 = coarse_hot(w, 0, u, topp, draw, f.P.top_p), h1 = coarse_hot(w, 1, u, topp, draw, f.P.top_p);
             // the hot factor, lowered when hot bins hold most candidates so
             // that a fine bin (a 1/kNB share of the weight) holds at most
             // kFineCap candidates, which the census can take
@@ -1465,6 +1525,7 @@ __device__ __noinline__ BigOut big_nucleus(Fin& f_in, const Filt& q_in, float y0
             const uint32_t W0 = block_excl_scan<kBlock>(w0c + w1c, f.tmp(), &wtot);
             e_lay()[2 * tid] = W0;
             e_lay()[2 * tid + 1] = W0 + w0c;
+            if (tid == kBlock - 1) e_lay()[kNB] = W0 + w0c + (kNB - 1u);
             vb.scale = static_cast<float>(kNB) / static_cast<float>(wtot);
             TSM_LDS_SYNC();
             eng_pass<EP_HIST>(f, q, vb, 0.0f);
@@ -1480,7 +1541,7 @@ __device__ __noinline__ BigOut big_nucleus(Fin& f_in, const Filt& q_in, float y0
         // NaN everywhere downstream (an infinite best value, or a NaN
         // candidate): total, acc and r are NaN, no step decides, and the
         // reference keeps every candidate and picks the last (sampler.rs:150)
-        if (len == 0) len = count_pass<kNucGroup>(f, q);
+        if (len == 0) len = count_pass(f, q);
         if (len <= kExactCap) {  // exact_finalize carries the NaNs as the reference does
             out.small = true;
             out.pick.keep = len;
@@ -1495,7 +1556,7 @@ __device__ __noinline__ BigOut big_nucleus(Fin& f_in, const Filt& q_in, float y0
         return out;
     }
     // total's (and the draw's) plans, sums and census
-    plan_sr(f, u, draw, topp);
+    plan_sr(f, u, draw, topp, 1.0 / (static_cast<double>(vb.vb.mul) * t));
     for (uint32_t i = tid; i < 4u * kNB / 32u; i += kBlock) {
         e_tie()[i] = 0u;
         e_tieb()[i] = 0u;
@@ -1670,10 +1731,11 @@ __device__ __noinline__ Pick reread_nucleus(Fin& f, uint32_t nallow, float u, co
     (void)nallow;
     const uint32_t tid = threadIdx.x;
     const RowMode& m = f.m;
+    pen_build(f);
     float mall = -INFINITY, mal = -INFINITY, mlo = INFINITY;
     {
         float la = -INFINITY, lb = -INFINITY, lc = INFINITY;
-        row_pass<2 * kNucGroup>(f, [&](uint32_t id, float x, float y) {
+        row_pass(f, [&](uint32_t id, float x, float y) {
             la = fmaxf(la, y);
             lc = fminf(lc, y);
             if (m.constrained && allowed_bit(f, id)) lb = fmaxf(lb, y);
@@ -1704,15 +1766,15 @@ __device__ __noinline__ Pick reread_nucleus(Fin& f, uint32_t nallow, float u, co
     q0.need_allowed = m.constrained;
     uint32_t n0 = 0xFFFFFFFFu;  // not counted
     if (m.constrained) {
-        n0 = count_pass<kNucGroup>(f, q0);
+        n0 = count_pass(f, q0);
         if (n0 == 0) {  // sampler.rs:211-221: every allowed id, by total_cmp
             q0.use_cut = false;
-            n0 = count_pass<kNucGroup>(f, q0);
+            n0 = count_pass(f, q0);
         }
     }
     Filt q1 = q0;
     if (m.want < f.n) {  // ranked.truncate(want)
-        if (n0 == 0xFFFFFFFFu) n0 = count_pass<kNucGroup>(f, q0);
+        if (n0 == 0xFFFFFFFFu) n0 = count_pass(f, q0);
         if (n0 > m.want) {
             q1.use_max = true;
             q1.max_comp = select_kth(f, q0, m.want);

@@ -877,6 +877,8 @@ __device__ __forceinline__ void nan_top_list(uint32_t* top_ids, float* top_lp, u
     }
 }
 
+// kNucleus: rows without top-k come here too (the lean kernel has none).
+template <bool kNucleus>
 __device__ __forceinline__ void finish_row(const SampleArgs& a, const Fin& f_in, const Targets tg0,
                                            const uint32_t nlp, const float lref, const double lsum, uint32_t nallow,
                                            uint32_t bufn) {
@@ -1025,8 +1027,8 @@ __device__ __forceinline__ void finish_row(const SampleArgs& a, const Fin& f_in,
     if (none_allowed) {
         // nothing allowed: argmax of the raw row, no draw (sampler.rs:139-141)
         pk.token = static_cast<uint32_t>(raw_best);
-    } else if (!m.topk) {
-        pk = reread_nucleus(f, nallow, u, dptr);
+    } else if (kNucleus && !m.topk) {
+        if constexpr (kNucleus) pk = reread_nucleus(f, nallow, u, dptr);
     } else if (!buf_ok) {
         const uint32_t len = reread_topk_list(f, nallow);
         pk = finish_list(f, len, u, dptr);
@@ -1976,7 +1978,7 @@ __device__ __noinline__ void finish_row_call(float lref, double lsum, uint32_t n
     const Targets tg0 = row_call()->tg0;
     const uint32_t nlp = row_call()->nlp, bufn = row_call()->bufn;
     TSM_LDS_SYNC();  // read by every thread before the finish reuses the area
-    finish_row(a, f, tg0, nlp, lref, lsum, nallow, bufn);
+    finish_row<false>(a, f, tg0, nlp, lref, lsum, nallow, bufn);
 }
 
 // One row of a sampling step.  kLean: the lean kernel, which takes only the
@@ -2585,7 +2587,7 @@ __device__ __forceinline__ void sample_row(const SampleArgs& a) {
         m.want <= kWaveList && nlp <= kWaveList) {
         if (finish_wave(a, f, tg0, nlp, lse.ref, lse.sum, nallow, bufn)) return;
     }
-    finish_row(a, f, tg0, nlp, lse.ref, lse.sum, nallow, bufn);
+    finish_row<true>(a, f, tg0, nlp, lse.ref, lse.sum, nallow, bufn);
     }
 }
 

@@ -95,6 +95,7 @@ struct Fin {
     const uint32_t* hist;
     uint32_t hlen, n;
     float u;  // the row's uniform draw (0 for distribution())
+    uint32_t pen_table = 0;  // 1: the penalized ids' counts are in the LDS table (pen_build)
     RowMode m;
     tsm_row_params P;
     __device__ __forceinline__ uint32_t* cnt() const { return reinterpret_cast<uint32_t*>(lds_base() + kOffCnt); }
@@ -142,86 +143,214 @@ __device__ __forceinline__ bool keep_el(const Fin& f, const Filt& q, uint32_t id
     return true;
 }
 
-// One re-read of the row in tiles of kReTile ids; fn(id, raw, penalized) for
-// every id.  The row is read as 16-byte blocks from the aligned address at or
-// below its start (ids outside the row are skipped; a block that reaches
-// before the row's first id or past its last is read element by element), two
-// blocks per thread per tile, with the next tile's blocks in flight while one
-// is processed.  Penalized rows count the history ids of each tile in LDS.
-template <int G = 1, class F>
-__device__ void row_pass(Fin& f, F&& fn) {
-    (void)G;
-    const uint32_t tid = threadIdx.x;
-    const uint32_t n = f.n;
-    const bool penal = f.m.penal;
-    const TSM_GLOBAL_AS float* rowp = global_as(f.rowp);
-    const uint32_t head = static_cast<uint32_t>((reinterpret_cast<uintptr_t>(f.rowp) >> 2) & 3u);
-    const TSM_GLOBAL_AS float* base = rowp - head;  // 16-byte aligned
-    const uint32_t span = head + n;         // aligned-base-relative end
-    const uint32_t nblk = (span + 3u) / 4u;  // blocks that hold row ids
-    const uint32_t full = span / 4u;         // blocks wholly before the row's end
-    constexpr uint32_t kTB = kReTile / 4u;  // blocks per tile
-    constexpr uint32_t kPer = kTB / kBlock;
-    static_assert(kPer * kBlock == kTB, "blocks per thread per tile");
+// ---- a re-read's penalties -----------------------------------------------------
+// The history's distinct ids and their counts in one word each, in an
+// open-addressing table over the tile-count area (built once per row, kept
+// through its re-reads): an element's count is then one bitmap bit away and a
+// table probe for the few ids whose bit is set, where counting each tile's
+// history ids anew took three barriers and a walk over the whole history every
+// 8192 ids.  Longer histories and rows past 2^20 ids keep the counting.
+constexpr uint32_t kPenSlots = 4096;
+constexpr uint32_t kPenCntBits = 12;
+constexpr uint32_t kPenEmpty = 0xFFFFFFFFu;
+static_assert(kPenSlots * 4 == kReTile * 2, "the table fills the tile-count area");
+static_assert(kHistFast < (1u << kPenCntBits) && kHistFast <= kPenSlots / 2, "counts fit a word, the table stays half empty");
+constexpr uint32_t kPenBitIds = 32768;  // ids the bitmap holds at a time (a pass moves it along the row)
+static_assert(kPenBitIds / 8 <= 2 * kSBins * 4, "the bitmap fits the stream's histograms");
+__device__ __forceinline__ uint32_t* pen_table() { return reinterpret_cast<uint32_t*>(lds_base() + kOffCnt); }
+__device__ __forceinline__ uint32_t* pen_bits() { return reinterpret_cast<uint32_t*>(lds_base() + kOffSHist); }
+__device__ __forceinline__ uint32_t pen_slot(uint32_t id) { return (id * 2654435761u) >> 20; }
+static_assert(kPenSlots == 4096, "pen_slot yields 12 bits");
+
+// Builds the table when the row's history fits it and sets f.pen_table.
+__device__ __noinline__ void pen_build(Fin& f) {
+    f.pen_table = f.m.penal && f.hlen <= kHistFast && f.n <= (1u << (32u - kPenCntBits)) - 1u ? 1u : 0u;
+    if (!f.pen_table) return;
+    const uint32_t tid = threadIdx.x, n = f.n, hc = f.hlen;
     const TSM_GLOBAL_AS uint32_t* hist = global_as(f.hist);
-    const uint32_t hc = min(f.hlen, TSM_MAX_HISTORY);
-    auto load_blk = [&](uint32_t j) -> float4 {
-        if (j < full && (j > 0u || head == 0u)) return load4(base + 4u * j);
-        float4 r = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (j < nblk) {
-            const uint32_t i0 = 4u * j;
-            if (i0 >= head && i0 < span) r.x = rowp[i0 - head];
-            if (i0 + 1u >= head && i0 + 1u < span) r.y = rowp[i0 + 1u - head];
-            if (i0 + 2u >= head && i0 + 2u < span) r.z = rowp[i0 + 2u - head];
-            if (i0 + 3u >= head && i0 + 3u < span) r.w = rowp[i0 + 3u - head];
+    TSM_LDS_SYNC();
+    for (uint32_t i = tid; i < kPenSlots; i += kBlock) pen_table()[i] = kPenEmpty;
+    TSM_LDS_SYNC();
+    for (uint32_t h = tid; h < hc; h += kBlock) {
+        const uint32_t id = hist[h];
+        if (id >= n) continue;
+        for (uint32_t s = pen_slot(id);; s = (s + 1u) & (kPenSlots - 1u)) {  // at most half the slots fill: ends
+            const uint32_t old = atomicCAS(&pen_table()[s], kPenEmpty, id << kPenCntBits | 1u);
+            if (old == kPenEmpty) break;
+            if (old >> kPenCntBits == id) {
+                atomicAdd(&pen_table()[s], 1u);
+                break;
+            }
         }
-        return r;
+    }
+    TSM_LDS_SYNC();
+}
+// Occurrences of an id that is in the table.
+__device__ __forceinline__ uint32_t pen_count(uint32_t id) {
+    uint32_t s = pen_slot(id), e = pen_table()[s];
+    while (e >> kPenCntBits != id && e != kPenEmpty) {
+        s = (s + 1u) & (kPenSlots - 1u);
+        e = pen_table()[s];
+    }
+    return e == kPenEmpty ? 0u : e & ((1u << kPenCntBits) - 1u);
+}
+
+// A value every lane of the wave holds (loaded through a reference to private
+// memory it would sit in a vector register, and each branch on it would be an
+// exec-mask branch): in a scalar register.
+__device__ __forceinline__ float wave_uniform_f(float v) { return __uint_as_float(wave_uniform(__float_as_uint(v))); }
+template <class T>
+__device__ __forceinline__ T* wave_uniform_p(T* p) {
+    const uint64_t v = reinterpret_cast<uint64_t>(p);
+    return reinterpret_cast<T*>(static_cast<uint64_t>(wave_uniform(static_cast<uint32_t>(v >> 32))) << 32 |
+                                wave_uniform(static_cast<uint32_t>(v)));
+}
+
+// One re-read of the row; fn4(id, m, x, y) for every four consecutive ids of an
+// aligned 16-byte block: the first one's id (below 0, wrapped, for a block that
+// reaches before the row), m's bit e set when id + e is in the row, raw values
+// and penalized ones.  Blocks wholly inside the row are read four per thread
+// and tile, with the next tile's four in flight while one is processed: two in
+// flight left every tile waiting for memory.  The blocks that reach past the
+// row's ends come last, read element by element.  Everything that is the same
+// for the whole workgroup is held in scalar registers; a pass over 151,936 ids
+// that finds their maximum went from 144 us to 46 us with both.
+template <class F>
+__device__ __forceinline__ void row_blocks(const Fin& f, F&& fn4) {
+    const uint32_t tid = threadIdx.x;
+    const uint32_t n = wave_uniform(f.n);
+    const bool table = wave_uniform(f.pen_table) != 0u, count = wave_uniform(f.m.penal ? 1u : 0u) != 0u && !table;
+    RowMode pm;  // what penalize() reads
+    pm.pen_rep = wave_uniform(f.m.pen_rep ? 1u : 0u) != 0u;
+    pm.pen_pf = wave_uniform(f.m.pen_pf ? 1u : 0u) != 0u;
+    tsm_row_params pp;
+    pp.repetition_penalty = wave_uniform_f(f.P.repetition_penalty);
+    pp.presence_penalty = wave_uniform_f(f.P.presence_penalty);
+    pp.frequency_penalty = wave_uniform_f(f.P.frequency_penalty);
+    const TSM_GLOBAL_AS float* rowp = global_as(wave_uniform_p(f.rowp));
+    const uint32_t head = wave_uniform(static_cast<uint32_t>((reinterpret_cast<uintptr_t>(f.rowp) >> 2) & 3u));
+    const TSM_GLOBAL_AS float* base = rowp - head;        // 16-byte aligned
+    const uint32_t first = head ? 1u : 0u;                // blocks [first, full) lie inside the row
+    const uint32_t full = (head + n) / 4u;
+    const uint32_t nin = full > first ? full - first : 0u;
+    constexpr uint32_t kPer = 4;
+    constexpr uint32_t kTB = kPer * kBlock;               // blocks per tile
+    constexpr uint32_t kSub = kReTile / 4u / kBlock;      // blocks per thread and counted stretch of the history
+    static_assert(kPer % kSub == 0 && kPenBitIds % (4u * kTB) == 0, "tiles hold whole counted stretches, bitmaps whole tiles");
+    const TSM_GLOBAL_AS uint32_t* hist = global_as(wave_uniform_p(f.hist));
+    const uint32_t hc = wave_uniform(min(f.hlen, TSM_MAX_HISTORY));
+    // past the last block the last one is read again (and its ids masked)
+    auto load_blk = [&](uint32_t i) __attribute__((always_inline)) -> float4 {
+        return load4(base + 4u * (first + min(i, nin - 1u)));
     };
+    // the blocks that reach past the row's ends, thread 0's and thread 1's in a
+    // round of their own: block 0 when the row starts inside it, and the block
+    // it ends inside
+    const uint32_t span = head + n;
+    const bool ends = head != 0u || (span & 3u) != 0u;
+    const uint32_t eblk = tid == 0u ? 0u : full;
+    const uint32_t ebits = (tid == 0u && head) || (tid == 1u && (span & 3u) && !(head && full == 0u)) ? 0xFu : 0u;
+    uint32_t em = 0;
+#pragma unroll
+    for (uint32_t e = 0; e < 4u; e++)
+        if (4u * eblk + e >= head && 4u * eblk + e < span) em |= 1u << e;
+    em &= ebits;
     float4 cur[kPer], nxt[kPer];
+    if (nin) {
 #pragma unroll
-    for (uint32_t k = 0; k < kPer; k++) cur[k] = load_blk(tid + k * kBlock);
-    const uint32_t ntiles = (nblk + kTB - 1u) / kTB;
-    for (uint32_t t = 0; t < ntiles; t++) {
-        if (t + 1u < ntiles) {
+        for (uint32_t k = 0; k < kPer; k++) cur[k] = load_blk(tid + k * kBlock);
+    }
+    const uint32_t ntiles = (nin + kTB - 1u) / kTB, rounds = ntiles + (ends ? 1u : 0u);
+    for (uint32_t t = 0; t < rounds; t++) {
+        const bool edge = t == ntiles;
+        const uint32_t i0 = t * kTB;  // the tile's first block
+        if (edge) {
+            float v[4];
 #pragma unroll
-            for (uint32_t k = 0; k < kPer; k++) nxt[k] = load_blk((t + 1u) * kTB + tid + k * kBlock);
+            for (uint32_t e = 0; e < 4u; e++) v[e] = (em >> e) & 1u ? rowp[4u * eblk + e - head] : 0.0f;
+            cur[0] = make_float4(v[0], v[1], v[2], v[3]);
+        } else if (t + 1u < ntiles) {
+#pragma unroll
+            for (uint32_t k = 0; k < kPer; k++) nxt[k] = load_blk(i0 + kTB + tid + k * kBlock);
         }
-        const uint32_t tb = t * kReTile;  // aligned-base-relative first id of the tile
-        if (penal) {
+        if (table && !edge && t % (kPenBitIds / (4u * kTB)) == 0u) {  // the next stretch's bitmap
             TSM_LDS_SYNC();
-            for (uint32_t i = tid; i < kReTile / 2; i += kBlock) f.cnt()[i] = 0;
+            for (uint32_t i = tid; i < kPenBitIds / 32u; i += kBlock) pen_bits()[i] = 0u;
             TSM_LDS_SYNC();
-            for (uint32_t h = tid; h < hc; h += kBlock) {
-                const uint32_t li = hist[h] + head - tb;
-                if (li < kReTile && hist[h] < n) atomicAdd(&f.cnt()[li >> 1], 1u << ((li & 1u) << 4));
+#pragma unroll
+            for (uint32_t k = 0; k < kPenSlots / kBlock; k++) {
+                const uint32_t e = pen_table()[tid + k * kBlock];
+                const uint32_t li = (e >> kPenCntBits) + head - 4u * (first + i0);
+                if (e != kPenEmpty && li < kPenBitIds) atomicOr(&pen_bits()[li >> 5], 1u << (li & 31u));
             }
             TSM_LDS_SYNC();
         }
+        // one copy of the work for the tile's blocks: unrolled, the larger
+        // passes no longer fit the instruction cache
+#pragma unroll 1
+        for (uint32_t k = 0; k < (edge ? 1u : kPer); k++) {
+            const uint32_t i = i0 + tid + k * kBlock;
+            static_assert(kPer == 4, "the choice below");
+            const float4 c01 = (k & 1u) ? cur[1] : cur[0], c23 = (k & 1u) ? cur[3] : cur[2];
+            const float4 c = (k & 2u) ? c23 : c01;
+            const float x[4] = {c.x, c.y, c.z, c.w};
+            float y[4] = {x[0], x[1], x[2], x[3]};
+            const uint32_t id0 = 4u * (edge ? eblk : first + i) - head;
+            const uint32_t m = edge ? em : (i < nin ? 0xFu : 0u);
+            if (table) {
+                const uint32_t li = 4u * (i & (kPenBitIds / 4u - 1u));
+                const uint32_t w = edge ? em : (pen_bits()[li >> 5] >> (li & 31u)) & 0xFu;
+                if (w != 0u) {
 #pragma unroll
-        for (uint32_t k = 0; k < kPer; k++) {
-            const uint32_t j = t * kTB + tid + k * kBlock;
-            if (j >= nblk) continue;
-            const float xv[4] = {cur[k].x, cur[k].y, cur[k].z, cur[k].w};
-#pragma unroll
-            for (uint32_t q = 0; q < 4u; q++) {
-                const uint32_t i = 4u * j + q;
-                if (i < head || i >= span) continue;
-                const float x = xv[q];
-                float y = x;
-                if (penal) {
-                    const uint32_t li = i - tb;
-                    const uint32_t c = (f.cnt()[li >> 1] >> ((li & 1u) << 4)) & 0xFFFFu;
-                    if (c) y = penalize(x, c, f.m, f.P);
+                    for (uint32_t e = 0; e < 4u; e++)
+                        if ((w >> e) & 1u) {
+                            const uint32_t c = pen_count(id0 + e);
+                            if (c) y[e] = penalize(x[e], c, pm, pp);
+                        }
                 }
-                fn(i - head, x, y);
+            } else if (count) {
+                // the stretch's first id from the aligned base; at the ends each
+                // thread's four ids have places of their own
+                const uint32_t tb = 4u * (first + i0 + k / kSub * kSub * kBlock);
+                if (k % kSub == 0u) {
+                    TSM_LDS_SYNC();
+                    for (uint32_t z = tid; z < kReTile / 2; z += kBlock) f.cnt()[z] = 0;
+                    TSM_LDS_SYNC();
+                    for (uint32_t h = tid; h < hc; h += kBlock) {
+                        const uint32_t at = hist[h] + head;  // aligned-base-relative
+                        if (hist[h] >= n) continue;
+                        const uint32_t li = !edge ? at - tb : at < 4u ? at : at >= 4u * full ? at - 4u * full + 4u : kReTile;
+                        if (li < kReTile) atomicAdd(&f.cnt()[li >> 1], 1u << ((li & 1u) << 4));
+                        if (edge && at < 4u && full == 0u)  // a row inside one block: thread 1's place too
+                            atomicAdd(&f.cnt()[(at + 4u) >> 1], 1u << (((at + 4u) & 1u) << 4));
+                    }
+                    TSM_LDS_SYNC();
+                }
+#pragma unroll
+                for (uint32_t e = 0; e < 4u; e++) {
+                    const uint32_t li = edge ? 4u * tid + e : id0 + e + head - tb;
+                    const uint32_t c = (f.cnt()[li >> 1] >> ((li & 1u) << 4)) & 0xFFFFu;
+                    if (c) y[e] = penalize(x[e], c, pm, pp);
+                }
             }
+            fn4(id0, m, x, y);
         }
-        if (t + 1u < ntiles) {
+        if (!edge) {
 #pragma unroll
             for (uint32_t k = 0; k < kPer; k++) cur[k] = nxt[k];
         }
     }
     TSM_LDS_SYNC();
+}
+
+// The same, fn(id, raw, penalized) for every id of the row.
+template <class F>
+__device__ __forceinline__ void row_pass(Fin& f, F&& fn) {
+    row_blocks(f, [&](uint32_t id, uint32_t m, const float (&x)[4], const float (&y)[4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; e++)
+            if ((m >> e) & 1u) fn(id + e, x[e], y[e]);
+    });
 }
 
 // Block-wide bitonic sort, ascending, of n u64 (n a power of two <= 4096).
@@ -250,10 +379,9 @@ __device__ __forceinline__ uint32_t pow2_ceil(uint32_t v) {
 }
 
 // Counts filtered elements (one pass).
-template <int G = 1>
 __device__ __forceinline__ uint32_t count_pass(Fin& f, const Filt& q) {
     uint32_t local = 0;
-    row_pass<G>(f, [&](uint32_t id, float x, float y) {
+    row_pass(f, [&](uint32_t id, float x, float y) {
         const uint64_t c = comp_of(q.order, id, x, y);
         if (keep_el(f, q, id, y, c)) local++;
     });
@@ -354,11 +482,10 @@ __device__ double block_excl_scan_f64(double v, double* tmp, double* total) {
 }
 
 // Gathers filtered elements' composites into gcomp (caller guarantees <= cap).
-template <int G = 1>
 __device__ __forceinline__ uint32_t gather_pass(Fin& f, const Filt& q, uint32_t cap) {
     if (threadIdx.x == 0) f.misc()[M_CNT] = 0;
     TSM_LDS_SYNC();
-    row_pass<G>(f, [&](uint32_t id, float x, float y) {
+    row_pass(f, [&](uint32_t id, float x, float y) {
         const uint64_t c = comp_of(q.order, id, x, y);
         if (keep_el(f, q, id, y, c)) {
             const uint32_t pos = atomicAdd(&f.misc()[M_CNT], 1u);
@@ -408,8 +535,6 @@ __device__ void sort_gathered(Fin& f, uint32_t n) {
     TSM_LDS_SYNC();
 }
 
-constexpr int kNucGroup = 4;  // loads in flight per thread in the nucleus passes
-
 // ---- value bins ------------------------------------------------------------------
 // bin(y) = floor((y0 - y) * mul), clamped to [0, kBins): (y0 - y) * mul is
 // monotone in y, so ascending bins visit the elements in (value desc) order
@@ -418,8 +543,7 @@ struct VBins {
     float y0, mul;
     __device__ __forceinline__ float pos(float y) const { return (y0 - y) * mul; }
     __device__ __forceinline__ uint32_t bin(float y) const {
-        const float d = pos(y);
-        return d >= static_cast<float>(kBins - 1) ? kBins - 1u : (d > 0.0f ? static_cast<uint32_t>(d) : 0u);
+        return static_cast<uint32_t>(fminf(fmaxf(pos(y), 0.0f), static_cast<float>(kBins - 1)));
     }
 };
 static_assert(kBins == 2 * kBlock, "two bins per thread");
@@ -614,6 +738,7 @@ __device__ Pick finish_list(Fin& f, uint32_t len, float u, const DistOut* dist) 
 // whole-vocabulary fallback (sampler.rs:192-222).  Leaves the ranked list in
 // ry/rid and returns its length.
 __device__ uint32_t reread_topk_list(Fin& f, uint32_t nallow) {
+    pen_build(f);
     uint32_t len = 0;
     if (!slow_topk_window(f, &len)) len = slow_fallback(f, nallow);
     return len;
@@ -623,7 +748,7 @@ __device__ uint32_t reread_topk_list(Fin& f, uint32_t nallow) {
 __device__ __noinline__ Pick nucleus_exact(Fin& f_in, const Filt& q_in, float u, const DistOut* dist) {
     Fin f = f_in;  // a private copy: its fields stay in registers across LDS atomics
     const Filt q = q_in;
-    const uint32_t g = gather_pass<kNucGroup>(f, q, kExactCap);
+    const uint32_t g = gather_pass(f, q, kExactCap);
     sort_gathered(f, g);
     return finish_list(f, g, u, dist);
 }
