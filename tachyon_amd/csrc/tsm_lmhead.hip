@@ -380,7 +380,9 @@ __global__ __launch_bounds__(T::kThreads) void lm_gemm_kernel(GemmArgs a) {
 //                      operands of the next kQ8Ring pairs in flight in a
 //                      register ring, issued in the order they are used.
 //                      Tiles by batch size (Q8Tile): a wave owns RB row
-//                      blocks x JB id blocks of 16; WR x WN waves.
+//                      blocks x JB id blocks of 16; WR x WN waves.  For
+//                      batches of up to 32 rows; the larger ones take
+//                      lm_q8_gemm32_kernel, below.
 constexpr uint32_t kQ8Block = 32;       // values per quantization block
 constexpr uint32_t kQ8Threads = 1024;   // prep kernel (one round of the quantization at dim 4096)
 constexpr uint32_t kQ8Stage = 4096;     // squares staged per round of the prep's fold
@@ -519,19 +521,9 @@ __global__ __launch_bounds__(kQ8Threads) void lm_q8_prep_kernel(Q8PrepArgs a) {
 // rows' scales of both blocks, from L2.  A ring of T::kRing slots: the loads
 // of pair p + kRing are issued as pair p is done, weights and activations
 // together, so the waits on the load counter (which retires loads in order)
-// never hold a load that is needed later than one still in flight.  With
-// kPaired (nb a multiple of 8, wscale 16-byte aligned) the ids' scales come
-// a round of kQ8SRound pairs at a time, one 16-byte load per id block (lane
-// group g: the scales of pairs 16t + 4g .. 16t + 4g + 3), passed to the
-// other lane groups with ds_bpermute: a 128-byte line of an id's scales is
-// read by two loads, not sixteen.  Otherwise two 2-byte loads per id block
-// and pair.
+// never hold a load that is needed later than one still in flight.  Two 2-byte
+// scale loads per id block and pair.
 constexpr uint32_t kQ8SRound = 16;
-constexpr uint32_t q8_lcm(uint32_t a, uint32_t b) {
-    uint32_t m = a;
-    while (m % b) m += a;
-    return m;
-}
 template <class T>
 struct Q8Slot {
     i32x4 bf[T::JB];
@@ -540,10 +532,9 @@ struct Q8Slot {
     f32x4 xs[T::RB][2];
 };
 
-template <class T, bool kPaired>
+template <class T>
 __global__ __launch_bounds__(T::kThreads) void lm_q8_gemm_kernel(Q8GemmArgs a) {
-    constexpr uint32_t RB = T::RB, JB = T::JB, R = T::kRing, U = q8_lcm(T::kRing, kQ8SRound);
-    static_assert(kQ8SRound == 16, "a round's scales: four pairs per lane group");
+    constexpr uint32_t RB = T::RB, JB = T::JB, R = T::kRing, U = T::kRing;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wid = tid >> 6;
     const uint32_t wr = wid % T::WR, wn = wid / T::WR;
     const uint32_t nb = a.dim / kQ8Block, np = (nb + 1u) / 2u, nrb = a.rows_pad / 16u;
@@ -586,10 +577,8 @@ __global__ __launch_bounds__(T::kThreads) void lm_q8_gemm_kernel(Q8GemmArgs a) {
 #pragma unroll
         for (uint32_t j = 0; j < JB; j++) {
             o.bf[j] = two || !upper ? *reinterpret_cast<const i32x4*>(wrow[j] + static_cast<size_t>(p) * 64u) : zi;
-            if (!kPaired) {
-                o.wsh[j][0] = wsrow[j][2u * p];
-                o.wsh[j][1] = two ? wsrow[j][2u * p + 1u] : 0u;
-            }
+            o.wsh[j][0] = wsrow[j][2u * p];
+            o.wsh[j][1] = two ? wsrow[j][2u * p + 1u] : 0u;
         }
 #pragma unroll
         for (uint32_t i = 0; i < RB; i++) {
@@ -597,26 +586,6 @@ __global__ __launch_bounds__(T::kThreads) void lm_q8_gemm_kernel(Q8GemmArgs a) {
             o.af[i] = rbok[i] ? *reinterpret_cast<const i32x4*>(abase[i] + static_cast<size_t>(p) * 1024u) : zi;
             o.xs[i][0] = rbok[i] ? *reinterpret_cast<const f32x4*>(sp) : zf;
             o.xs[i][1] = rbok[i] && two ? *reinterpret_cast<const f32x4*>(sp + 16) : zf;
-        }
-    };
-    // kPaired: the scales of pairs 16t .. 16t + 15, lane group g holding
-    // pairs 16t + 4g .. 16t + 4g + 3 (dword d: pair 16t + 4g + d, its two
-    // blocks' scales); np is a multiple of 4, so a group's pairs all exist
-    // or none do
-    auto load_s = [&](u32x4 (&sc)[JB], uint32_t t) {
-        const uint32_t p = kQ8SRound * t + 4u * (lane >> 4);
-#pragma unroll
-        for (uint32_t j = 0; j < JB; j++)
-            sc[j] = p < np ? *reinterpret_cast<const u32x4*>(wsrow[j] + 2u * p) : u32x4{0u, 0u, 0u, 0u};
-    };
-    // the scales of pair 16t + u (u the same in every lane) from lane group u / 4
-    auto take_s = [&](Q8Slot<T>& o, const u32x4 (&sc)[JB], uint32_t u) {
-#pragma unroll
-        for (uint32_t j = 0; j < JB; j++) {
-            const uint32_t v = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(
-                static_cast<int>(4u * ((lane & 15u) + 16u * (u >> 2))), static_cast<int>(sc[j][u & 3u])));
-            o.wsh[j][0] = v & 0xFFFFu;
-            o.wsh[j][1] = v >> 16;
         }
     };
     auto scale_add_one = [&](const Q8Slot<T>& o, uint32_t h) {
@@ -637,25 +606,16 @@ __global__ __launch_bounds__(T::kThreads) void lm_q8_gemm_kernel(Q8GemmArgs a) {
         }
     };
     Q8Slot<T> ring[R];
-    u32x4 scur[JB], snext[JB];
-    if (kPaired) load_s(snext, 0);
 #pragma unroll
     for (uint32_t u = 0; u < R; u++)
         if (u < np) load(ring[u], u);
-    // U pairs a round (a multiple of the ring and of the scale round), so
-    // every slot and lane group below is fixed at compile time
+    // a ring of pairs a round, so every slot below is fixed at compile time
     for (uint32_t p0 = 0; p0 < np; p0 += U) {
 #pragma unroll
         for (uint32_t u = 0; u < U; u++) {
             const uint32_t p = p0 + u;
             if (p >= np) break;
-            if (kPaired && u % kQ8SRound == 0) {
-#pragma unroll
-                for (uint32_t j = 0; j < JB; j++) scur[j] = snext[j];
-                if (p + kQ8SRound < np) load_s(snext, p / kQ8SRound + 1u);
-            }
             Q8Slot<T>& o = ring[u % R];
-            if (kPaired) take_s(o, scur, u % kQ8SRound);
             // the pair's blocks in order
             scale_add_one(o, 0);
             if (2u * p + 1u < nb) scale_add_one(o, 1);
@@ -836,31 +796,242 @@ __global__ __launch_bounds__(T::kThreads) void lm_q8_gemm_line_kernel(Q8GemmArgs
     }
 }
 
-// With paired scales batches of up to 32 rows take the whole-line kernel
-// (its own tiles: 16 or 32 rows x 128 ids), the others the pair-at-a-time
-// kernel.
-template <class T, bool kPaired>
-void launch_q8_gemm(const Q8GemmArgs& g, hipStream_t st) {
-    const dim3 grid((g.vocab + T::kIds - 1u) / T::kIds, (g.rows_pad + T::kRows - 1u) / T::kRows);
-    if constexpr (kPaired && T::JB == 2u) hipLaunchKernelGGL((lm_q8_gemm_line_kernel<T>), grid, dim3(T::kThreads), 0, st, g);
-    else hipLaunchKernelGGL((lm_q8_gemm_kernel<T, kPaired>), grid, dim3(T::kThreads), 0, st, g);
+// ---- batches of more than 32 rows ------------------------------------------
+// The f32 scaling bounds these: per row, id and block the integer dot times the
+// weight block's scale, times the row block's scale, added in block order.
+// Three VALU operations do it where converting, two products and a sum took
+// four (19.9 G lane operations for 256 x 151,936 x 128, 507 us of issue): the
+// MFMA starts from the integer 0x4B400000, so that a dot s leaves it as the
+// f32 12582912 + s (|s| <= 2^19), and fma(12582912 + s, w, -12582912 w) rounds
+// s w once, as the product does; -12582912 w is exact for an f16 w.  Only the
+// sign of a zero dot's product is lost (+0 where w's sign would make -0), which
+// shows only where every term of a logit is zero: a logit that ends as +0 is
+// computed again step by step (q8_exact).
+//
+// A block is the 32 values of one v_mfma_i32_32x32x32_i8, so no lane group is
+// masked away.  A wave owns 64 rows x 32 JB ids (2 x JB tiles, 32 JB
+// accumulators a lane), WR waves lie along the rows, WN along the ids.  A step is a
+// chunk of 4 blocks: 128 contiguous bytes of each weight row, its scales (as
+// w and -12582912 w) and the rows' scales are staged in LDS, double-buffered,
+// one barrier a chunk, with the loads of the chunk after the next in flight;
+// the activations go from L2 into registers two blocks ahead.
+constexpr uint32_t kQ8Chunk = 4;
+constexpr uint32_t kQ8WStride = 32 * kQ8Chunk + 16;  // LDS bytes per weight row (16 B pad: no bank conflicts)
+constexpr float kQ8Magic = 12582912.0f;
+typedef int i32x16 __attribute__((ext_vector_type(16)));
+
+// One logit as dot_q8_with adds it up.
+__device__ __noinline__ float q8_exact(const int8_t* aq, const float* as, const int8_t* w, const uint16_t* ws,
+                                       uint32_t nb) {
+    // aq: block 0 of the row in its 16-row unit, 512 bytes a block; as: 16 floats a block
+    float acc = -0.0f;
+#pragma unroll 1
+    for (uint32_t b = 0; b < nb; b++) {
+        int s = 0;
+#pragma unroll 1
+        for (uint32_t k = 0; k < kQ8Block; k++)
+            s += static_cast<int>(aq[512u * b + 256u * (k >> 4) + (k & 15u)]) * static_cast<int>(w[kQ8Block * b + k]);
+        acc = acc + static_cast<float>(s) * q8_f16(ws[b]) * as[16u * b];
+    }
+    return acc;
 }
 
-template <bool kPaired>
-void launch_q8_tiles(const Q8GemmArgs& g, hipStream_t st) {
-    // tiles by batch (rows x ids): 16 x 128 (whole lines) or 16 x 256, 32 x 128 (whole lines) or 32 x 256,
-    // 64 x 256, 128 x 128, 256 x 64
+// kWide: nb a multiple of 4 and wscale 8-byte aligned (a chunk's scales of an
+// id are one 8-byte load; otherwise four 2-byte loads).
+template <uint32_t JB, uint32_t WR, uint32_t WN, bool kWide>
+__global__ __launch_bounds__(64 * WR * WN, 2) void lm_q8_gemm32_kernel(Q8GemmArgs a) {
+    constexpr uint32_t kThreads = 64u * WR * WN, kRows = 64u * WR, kIds = 32u * JB * WN;
+    constexpr uint32_t kWLoads = kIds * 2u * kQ8Chunk / kThreads;  // 16-byte weight loads per thread and chunk
+    constexpr uint32_t kXLoads = kRows * kQ8Chunk / 4u;            // 16-byte row scale loads per chunk
+    static_assert(kWLoads * kThreads == kIds * 2u * kQ8Chunk && kXLoads <= kThreads, "loads per thread");
+    static_assert(kThreads % kIds == 0, "a thread per id");
+    __shared__ __attribute__((aligned(16))) uint8_t wbuf[2][kIds * kQ8WStride];
+    __shared__ __attribute__((aligned(16))) float xbuf[2][kQ8Chunk][kRows];
+    __shared__ __attribute__((aligned(16))) float2 sbuf[2][kQ8Chunk][kIds];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wid = tid >> 6;
+    const uint32_t wr = wid % WR, wn = wid / WR, half = lane >> 5;
+    const uint32_t nb = a.dim / kQ8Block, nb2 = (nb + 1u) / 2u * 2u;  // blocks, and a unit's places for them
+    const uint32_t units = a.rows_pad / 16u, nc = (nb + kQ8Chunk - 1u) / kQ8Chunk;
+    const uint32_t r0 = blockIdx.y * kRows, n0 = blockIdx.x * kIds;
+    // this thread's weight loads: 8 threads to a row's 128 bytes; ids past the
+    // vocabulary and blocks past the row read the last ones again
+    const int8_t* wp[kWLoads];
+    uint32_t wo[kWLoads];
+#pragma unroll
+    for (uint32_t q = 0; q < kWLoads; q++) {
+        const uint32_t id = (tid >> 3) + kThreads / 8u * q;
+        wp[q] = a.wq + static_cast<size_t>(min(n0 + id, a.vocab - 1u)) * a.dim + 16u * (tid & 1u);
+        wo[q] = id * kQ8WStride + 16u * (tid & 7u);
+    }
+    const uint32_t wblk = (tid >> 1) & 3u;  // the block of the chunk this thread's loads lie in
+    // scales: a thread takes one id's four
+    const uint16_t* sp = a.ws + static_cast<size_t>(min(n0 + tid % kIds, a.vocab - 1u)) * nb;
+    const bool takes_s = tid < kIds;
+    // row scales: rows 4 x .. 4 x + 3 of the workgroup's, block tid / (kRows / 4) of the chunk
+    const uint32_t xrow = 4u * (tid % (kRows / 4u)), xblk = tid / (kRows / 4u);
+    const bool takes_x = tid < kXLoads;
+    const uint32_t xunit = min((r0 + xrow) >> 4, units - 1u);
+    // activations: row 32 i + (lane & 31) of the wave's 64, bytes 16 half of a block
+    const int8_t* ap[2];
+#pragma unroll
+    for (uint32_t i = 0; i < 2u; i++) {
+        const uint32_t u = min((r0 + 64u * wr + 32u * i + (lane & 16u)) >> 4, units - 1u);
+        ap[i] = a.aq + static_cast<size_t>(u) * nb2 * 512u + (lane & 15u) * 16u + 256u * half;
+    }
+    i32x4 wreg[kWLoads];
+    uint32_t sreg[2] = {0u, 0u};
+    f32x4 xreg = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto fetch = [&](uint32_t c) __attribute__((always_inline)) {
+        const uint32_t b0 = kQ8Chunk * c;
+#pragma unroll
+        for (uint32_t q = 0; q < kWLoads; q++)
+            wreg[q] = *reinterpret_cast<const i32x4*>(wp[q] + 32u * min(b0 + wblk, nb - 1u));
+        if (takes_s) {
+            if (kWide) {
+                const uint2 v = *reinterpret_cast<const uint2*>(sp + b0);
+                sreg[0] = v.x;
+                sreg[1] = v.y;
+            } else {
+                sreg[0] = sp[min(b0, nb - 1u)] | static_cast<uint32_t>(sp[min(b0 + 1u, nb - 1u)]) << 16;
+                sreg[1] = sp[min(b0 + 2u, nb - 1u)] | static_cast<uint32_t>(sp[min(b0 + 3u, nb - 1u)]) << 16;
+            }
+        }
+        if (takes_x)
+            xreg = *reinterpret_cast<const f32x4*>(a.as + (static_cast<size_t>(xunit) * nb + min(b0 + xblk, nb - 1u)) * 16u +
+                                                   (xrow & 15u));
+    };
+    auto stage = [&](uint32_t buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t q = 0; q < kWLoads; q++) *reinterpret_cast<i32x4*>(&wbuf[buf][wo[q]]) = wreg[q];
+        if (takes_s)
+#pragma unroll
+            for (uint32_t t = 0; t < kQ8Chunk; t++) {
+                const float w = q8_f16((sreg[t >> 1] >> (16u * (t & 1u))) & 0xFFFFu);
+                sbuf[buf][t][tid] = make_float2(w, -kQ8Magic * w);
+            }
+        if (takes_x) *reinterpret_cast<f32x4*>(&xbuf[buf][xblk][xrow]) = xreg;
+    };
+    f32x4 acc[2][JB][4];
+#pragma unroll
+    for (uint32_t i = 0; i < 2u; i++)
+#pragma unroll
+        for (uint32_t j = 0; j < JB; j++)
+#pragma unroll
+            for (uint32_t g = 0; g < 4u; g++) acc[i][j][g] = f32x4{-0.0f, -0.0f, -0.0f, -0.0f};  // Rust's f32 sum starts at -0.0
+    i32x16 magic;
+#pragma unroll
+    for (int e = 0; e < 16; e++) magic[e] = 0x4B400000;
+    i32x4 af[2][2];  // ring: blocks t and t + 1
+#pragma unroll
+    for (uint32_t t = 0; t < 2u; t++)
+#pragma unroll
+        for (uint32_t i = 0; i < 2u; i++)
+            af[t][i] = *reinterpret_cast<const i32x4*>(ap[i] + 512u * min(t, nb - 1u));
+    fetch(0);
+    stage(0);
+    fetch(min(1u, nc - 1u));
+    __syncthreads();
+    for (uint32_t c = 0; c < nc; c++) {
+        // every wave is done with buffer (c + 1) & 1 (chunk c - 1)
+        stage((c + 1u) & 1u);
+        const uint8_t* wb = &wbuf[c & 1u][(32u * JB * wn + (lane & 31u)) * kQ8WStride + 16u * half];
+#pragma unroll
+        for (uint32_t t = 0; t < kQ8Chunk; t++) {
+            const uint32_t b = kQ8Chunk * c + t;
+            if (b >= nb) break;
+            i32x4 bf[JB];
+            float2 w[JB];
+#pragma unroll
+            for (uint32_t j = 0; j < JB; j++) {
+                bf[j] = *reinterpret_cast<const i32x4*>(wb + 32u * j * kQ8WStride + 32u * t);
+                w[j] = sbuf[c & 1u][t][32u * JB * wn + 32u * j + (lane & 31u)];
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < 2u; i++) {
+                i32x16 sm[JB];
+#pragma unroll
+                for (uint32_t j = 0; j < JB; j++)
+                    sm[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[t & 1u][i], bf[j], magic, 0, 0, 0);
+                // lane: id lane & 31, rows 8 g + 4 half + e of the tile
+#pragma unroll
+                for (uint32_t g = 0; g < 4u; g++) {
+                    const f32x4 xs = *reinterpret_cast<const f32x4*>(&xbuf[c & 1u][t][64u * wr + 32u * i + 8u * g + 4u * half]);
+#pragma unroll
+                    for (uint32_t j = 0; j < JB; j++)
+#pragma unroll
+                        for (uint32_t e = 0; e < 4u; e++)
+                            acc[i][j][g][e] = acc[i][j][g][e] +
+                                              __builtin_fmaf(__int_as_float(sm[j][4u * g + e]), w[j].x, w[j].y) * xs[e];
+                }
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < 2u; i++)
+                af[t & 1u][i] = *reinterpret_cast<const i32x4*>(ap[i] + 512u * min(b + 2u, nb - 1u));
+            if (t == 0u) fetch(min(c + 2u, nc - 1u));  // after the activations' loads: those are waited for first
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < 2u; i++)
+#pragma unroll
+        for (uint32_t g = 0; g < 4u; g++)
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; e++) {
+                const uint32_t row = r0 + 64u * wr + 32u * i + 8u * g + 4u * half + e;
+                if (row >= a.rows) continue;
+#pragma unroll
+                for (uint32_t j = 0; j < JB; j++) {
+                    const uint32_t id = n0 + 32u * JB * wn + 32u * j + (lane & 31u);
+                    if (id >= a.vocab) continue;
+                    float v = acc[i][j][g][e];
+                    if (__float_as_uint(v) == 0u)
+                        v = q8_exact(a.aq + static_cast<size_t>(row >> 4) * nb2 * 512u + (row & 15u) * 16u,
+                                     a.as + static_cast<size_t>(row >> 4) * nb * 16u + (row & 15u),
+                                     a.wq + static_cast<size_t>(id) * a.dim, a.ws + static_cast<size_t>(id) * nb, nb);
+                    a.logits[static_cast<size_t>(row) * a.ld + id] = v;
+                }
+            }
+}
+
+template <uint32_t JB, uint32_t WR, uint32_t WN>
+void launch_q8_gemm32(const Q8GemmArgs& g, hipStream_t st) {
+    const dim3 grid((g.vocab + 32u * JB * WN - 1u) / (32u * JB * WN), (g.rows_pad + 64u * WR - 1u) / (64u * WR));
+    const bool wide = (g.dim / kQ8Block) % kQ8Chunk == 0 && (reinterpret_cast<uintptr_t>(g.ws) & 7u) == 0;
+    if (wide) hipLaunchKernelGGL((lm_q8_gemm32_kernel<JB, WR, WN, true>), grid, dim3(64u * WR * WN), 0, st, g);
+    else hipLaunchKernelGGL((lm_q8_gemm32_kernel<JB, WR, WN, false>), grid, dim3(64u * WR * WN), 0, st, g);
+}
+
+// Batches of up to 32 rows take the whole-line kernel when a round's scales of
+// an id are 16-byte loads (`paired`: dim a multiple of 256, wscale 16-byte
+// aligned), else the pair-at-a-time kernel; larger ones the 32-value blocks, in
+// the tile that holds them (rows x ids): 64 x 128, 128 x 64, 256 x 128.
+// Measured at dim 4096, vocab 151,936, against the pair-at-a-time kernel's
+// tiles before: 48 rows 236 us (381), 128 rows 334 (569), 256 rows 543 (1050);
+// 32 rows 222 with whole lines, 232 with the 64-row tile.  Two id tiles a wave
+// at 64 rows leave one wave a SIMD (348 us); one at 256 rows reads the row
+// scales twice as often from LDS (614).
+template <class T, bool kLine>
+void launch_q8_gemm(const Q8GemmArgs& g, hipStream_t st) {
+    const dim3 grid((g.vocab + T::kIds - 1u) / T::kIds, (g.rows_pad + T::kRows - 1u) / T::kRows);
+    if constexpr (kLine) hipLaunchKernelGGL((lm_q8_gemm_line_kernel<T>), grid, dim3(T::kThreads), 0, st, g);
+    else hipLaunchKernelGGL((lm_q8_gemm_kernel<T>), grid, dim3(T::kThreads), 0, st, g);
+}
+
+void launch_q8_tiles(const Q8GemmArgs& g, bool paired, hipStream_t st) {
     const uint32_t rp = g.rows_pad;
     if (rp <= 16u) {
-        if constexpr (kPaired) launch_q8_gemm<Q8Tile<1, 2, 1, 4>, true>(g, st);
+        if (paired) launch_q8_gemm<Q8Tile<1, 2, 1, 4>, true>(g, st);
         else launch_q8_gemm<Q8Tile<1, 4, 1, 4>, false>(g, st);
     } else if (rp <= 32u) {
-        if constexpr (kPaired) launch_q8_gemm<Q8Tile<2, 2, 1, 4>, true>(g, st);
+        if (paired) launch_q8_gemm<Q8Tile<2, 2, 1, 4>, true>(g, st);
         else launch_q8_gemm<Q8Tile<2, 4, 1, 4>, false>(g, st);
+    } else if (rp <= 64u) {
+        launch_q8_gemm32<1, 1, 4>(g, st);
+    } else if (rp <= 128u) {
+        launch_q8_gemm32<1, 2, 2>(g, st);
+    } else {
+        launch_q8_gemm32<2, 4, 2>(g, st);
     }
-    else if (rp <= 64u) launch_q8_gemm<Q8Tile<2, 4, 2, 4>, kPaired>(g, st);
-    else if (rp <= 128u) launch_q8_gemm<Q8Tile<2, 4, 4, 2>, kPaired>(g, st);
-    else launch_q8_gemm<Q8Tile<2, 4, 8, 1>, kPaired>(g, st);
 }
 
 void set_err(char* err, size_t errlen, const char* fmt, ...) {
@@ -1012,12 +1183,8 @@ int tsm_lm_head_q8(void* stream, const float* x, uint32_t x_stride, const float*
     g.dim = dim;
     g.vocab = vocab;
     g.ld = ld;
-    // the weight scales 16 pairs at a time when dim is a multiple of 256 and
-    // wscale 16-byte aligned, else 2 bytes a pair
-    if ((dim / tsm::lm::kQ8Block) % 8u == 0 && (reinterpret_cast<uintptr_t>(wscale) & 15u) == 0)
-        tsm::lm::launch_q8_tiles<true>(g, st);
-    else
-        tsm::lm::launch_q8_tiles<false>(g, st);
+    const bool paired = (dim / tsm::lm::kQ8Block) % 8u == 0 && (reinterpret_cast<uintptr_t>(wscale) & 15u) == 0;
+    tsm::lm::launch_q8_tiles(g, paired, st);
     e = hipGetLastError();
     if (e != hipSuccess) return set_err(err, errlen, "gemm launch failed: %s", hipGetErrorString(e)), 1;
     return 0;
