@@ -117,7 +117,6 @@ enum : uint32_t {  // e_sc() words
     SC_NAN = 2,     // a candidate is NaN
     SC_KLO = 3,     // predicted top-p bins: first, last
     SC_KHI = 4,
-    SC_NRUNS = 5,   // runs of the current census
     SC_RES = 6,     // walk: result, next bin, position, run, index within run, x bits
     SC_B = 7,
     SC_POS = 8,
@@ -371,29 +370,17 @@ __device__ uint32_t census_finish(const FBins& vb, float t) {
             e_rbin()[fin[k]] = fb[k];
             e_runp()[fin[k]] = fp[k];
         }
-    if (tid == 0) e_sc()[SC_NRUNS] = total;
     TSM_LDS_SYNC();
     return total;
 }
 
-// The first run whose bin is >= b (or > b with `after`): a 64-way search in
-// two steps (each lane tests one position).  Wave-uniform; every lane of the
-// wave takes part.
-__device__ __forceinline__ uint32_t runs_bound(uint32_t b, uint32_t nruns, bool after) {
-    const uint32_t lane = lane_id();
-    auto below = [&](uint32_t pos) { return pos < nruns && (after ? e_rbin()[pos] <= b : e_rbin()[pos] < b); };
-    static_assert(kHS <= 64u * 64u, "two 64-way steps cover the runs");
-    // step 1: blocks of 64 runs; lane l tests the last run of block l
-    const uint32_t nb1 = static_cast<uint32_t>(__popcll(wave_ballot(below(lane * 64u + 63u))));
-    const uint32_t base = nb1 * 64u;  // runs before base are all below
-    const uint32_t nb2 = static_cast<uint32_t>(__popcll(wave_ballot(below(base + lane))));
-    const uint32_t r = base + nb2;
-    return r < nruns ? r : nruns;
-}
-// First run of bin b and the end of its runs.
-__device__ __forceinline__ void runs_of(uint32_t b, uint32_t nruns, uint32_t* r0, uint32_t* r1) {
-    *r0 = runs_bound(b, nruns, false);
-    *r1 = runs_bound(b, nruns, true);
+// First run of a censused bin b and the end of its runs: census_finish leaves
+// each bucket's runs in its place, and e_bcnt the buckets' ends.
+__device__ __forceinline__ void runs_of(uint32_t b, uint32_t* r0, uint32_t* r1) {
+    const uint32_t ci = req_rank(b);
+    const uint32_t lo = e_bcnt()[ci ? ci - 1u : 0u];
+    *r0 = ci ? lo : 0u;
+    *r1 = e_bcnt()[ci];
 }
 
 // ---- stepping one run of equal terms ----------------------------------------
@@ -537,8 +524,7 @@ __device__ uint32_t walk_runs(Walk& w, uint32_t r0, uint32_t r1, float T, float 
 // whose sums also count candidates past it).  Total's walk records the fold
 // value and position at every bin start.
 template <int K, int kB = 0>
-__device__ uint32_t walk_bins(Walk& w, uint32_t bend, uint32_t nruns, float T, float thr, uint32_t force,
-                              uint32_t lim) {
+__device__ uint32_t walk_bins(Walk& w, uint32_t bend, float T, float thr, uint32_t force, uint32_t lim) {
     constexpr bool sub = K == FK_R;
     const uint32_t lane = lane_id();
     while (w.b < bend) {
@@ -570,33 +556,40 @@ __device__ uint32_t walk_bins(Walk& w, uint32_t bend, uint32_t nruns, float T, f
             uint32_t nj[kBL], cj[kBL];
             bool okj[kBL];
             uint32_t ln = 0, lc = 0, tmask = 0;  // tmask: the lane's summable bins holding a tie
+            // every word of the lane's bins first, whatever the plans turn out
+            // to say: one wait for LDS instead of one a bin and condition (with
+            // the runs found by their bucket: 60 -> 40 us for total's two walks
+            // of a row, 80 -> 60 us for the draw's)
+            uint32_t pj[kBL], s0[kBL], s1[kBL], t0[kBL], t1[kBL], a0[kBL], a1[kBL];
+#pragma unroll
+            for (uint32_t j = 0; j < kBL; j++) {
+                const uint32_t b = min(bl + j, kNB - 1u), i0 = slot0(K) * kNB + b, i1 = i0 + kNB;
+                nj[j] = e_cnt()[b];
+                pj[j] = e_plan()[b];
+                s0[j] = e_sum(slot0(K))[b];
+                s1[j] = e_sum(slot0(K) + 1u)[b];
+                t0[j] = e_tie()[i0 >> 5] >> (i0 & 31u);
+                t1[j] = e_tie()[i1 >> 5] >> (i1 & 31u);
+                a0[j] = e_tieb()[i0 >> 5] >> (i0 & 31u);
+                a1[j] = e_tieb()[i1 >> 5] >> (i1 & 31u);
+            }
 #pragma unroll
             for (uint32_t j = 0; j < kBL; j++) {
                 const uint32_t b = bl + j;
-                uint32_t n = 0;
-                bool ok = b < bend;  // past bend: the end marker
-                uint32_t c = 0;
-                if (ok) {
-                    n = e_cnt()[b];
-                    if (n) {
-                        const uint32_t pw = e_plan()[b];
-                        const int g0 = static_cast<int>((pw >> plan_shift(K)) & 0xFFu) - 128;
-                        uint32_t slot = 0xFFFFFFFFu;
-                        if (!(pw & plan_must(K)) && (K != FK_R || (pw & PF_R))) {
-                            if (e == g0) slot = slot0(K);
-                            else if (e == g0 + 1 && (pw & plan_two(K))) slot = slot0(K) + 1u;
-                        }
-                        // exact walks step through a bin with a tie; bound walks
-                        // take its lower (kB 1) or upper (kB 2) end
-                        ok = slot != 0xFFFFFFFFu && b != force &&
-                             (kB == 0 ? !tie_bit(slot, b) : !bad_bit(slot, b));
-                        if (ok) {
-                            const bool tie = kB != 0 && tie_bit(slot, b);
-                            c = min(e_sum(slot)[b], 1u << 25) + (kB == 2 && tie ? 1u : 0u);
-                            if (tie) tmask |= 1u << j;
-                        }
-                    }
-                }
+                const uint32_t n = b < bend ? nj[j] : 0u, pw = pj[j];
+                // the bin's sum for the fold's grid, if it has one
+                const int g0 = static_cast<int>((pw >> plan_shift(K)) & 0xFFu) - 128;
+                const bool planned = !(pw & plan_must(K)) && (K != FK_R || (pw & PF_R));
+                const bool low = planned && e == g0, high = planned && e == g0 + 1 && (pw & plan_two(K));
+                const bool tie = ((high ? t1[j] : t0[j]) & 1u) != 0u, bad = ((high ? a1[j] : a0[j]) & 1u) != 0u;
+                // exact walks step through a bin with a tie; bound walks take its
+                // lower (kB 1) or upper (kB 2) end
+                bool ok = (low || high) && b != force && (kB == 0 ? !tie : !bad);
+                uint32_t c = min(high ? s1[j] : s0[j], 1u << 25) + (kB == 2 && tie ? 1u : 0u);
+                const bool take = ok && n != 0u;
+                if (kB != 0 && take && tie) tmask |= 1u << j;
+                c = take ? c : 0u;
+                ok = b < bend && (ok || n == 0u);  // past bend: the end marker; an empty bin passes
                 // past 2^25 units a bin leaves the binade anyway: the clamps keep
                 // the prefix sums in 32 bits
                 cj[j] = min(c, 1u << 25);
@@ -669,7 +662,7 @@ __device__ uint32_t walk_bins(Walk& w, uint32_t bend, uint32_t nruns, float T, f
             const uint32_t bb = w.b;
             if (!bit_of(e_cpl(), bb)) return W_NEED;
             uint32_t r0, r1;
-            runs_of(bb, nruns, &r0, &r1);
+            runs_of(bb, &r0, &r1);
             const uint32_t res = walk_runs<K>(w, r0, r1, T, thr, lim);
             if (res == W_DECIDED) return res;
             w.b = bb + 1u;
@@ -1144,9 +1137,8 @@ __device__ __noinline__ uint32_t run_walk(Fin& f_in, const Filt& q_in, const FBi
     uint32_t last_from = kNoBin;
     bool alone = false;
     for (;;) {
-        const uint32_t nruns = e_sc()[SC_NRUNS];
         if (tid < kWave) {
-            const uint32_t res = walk_bins<K, kB>(w, bend, nruns, T, thr, force, lim);
+            const uint32_t res = walk_bins<K, kB>(w, bend, T, thr, force, lim);
             if (tid == 0) {
                 e_sc()[SC_RES] = res;
                 e_sc()[SC_B] = w.b;
@@ -1214,11 +1206,10 @@ __device__ __noinline__ uint32_t run_walk2(Fin& f_in, const Filt& q_in, const FB
     uint32_t from0 = kNoBin, from1 = kNoBin;  // the bin each walk last asked the census for
     bool alone = false;
     for (;;) {
-        const uint32_t nruns = e_sc()[SC_NRUNS];
         if (wid < 2u && (wid == 0u ? r0 : r1) == W_NEED) {
             Walk w = wid == 0u ? w0 : w1;
-            const uint32_t res = wid == 0u ? walk_bins<K, 1>(w, bend, nruns, T, thr, force, lim)
-                                           : walk_bins<K, 2>(w, bend, nruns, T, thr, force, lim);
+            const uint32_t res = wid == 0u ? walk_bins<K, 1>(w, bend, T, thr, force, lim)
+                                           : walk_bins<K, 2>(w, bend, T, thr, force, lim);
             if (lane_id() == 0) {
                 uint32_t* o = e_sc() + kSc2 + 7u * wid;
                 o[0] = res;
@@ -1285,9 +1276,9 @@ __device__ __noinline__ uint32_t run_walk2(Fin& f_in, const Filt& q_in, const FB
 
 // The kept candidate at position pos (0-based, pos < kept count) when no step
 // of the draw decides: its run and index within the run, from bin lb's runs.
-__device__ __forceinline__ bool locate(uint32_t lb, uint32_t pos, uint32_t nruns, uint32_t* run, uint32_t* within) {
+__device__ __forceinline__ bool locate(uint32_t lb, uint32_t pos, uint32_t* run, uint32_t* within) {
     uint32_t r0, r1;
-    runs_of(lb, nruns, &r0, &r1);
+    runs_of(lb, &r0, &r1);
     uint32_t at = e_pstart()[lb];
     for (uint32_t j = r0; j < r1; j++) {
         const uint32_t m = e_hcnt()[j];
@@ -1649,7 +1640,7 @@ __device__ __noinline__ BigOut big_nucleus(Fin& f_in, const Filt& q_in, float y0
                 wm.b = kb;
                 wm.pos = e_pstart()[kb];
                 uint32_t r0, r1;
-                runs_of(kb, e_sc()[SC_NRUNS], &r0, &r1);
+                runs_of(kb, &r0, &r1);
                 walk_runs<FK_S>(wm, r0, r1, 0.0f, 0.0f, keep);
                 if (tid == 0) e_sc()[SC_X] = __float_as_uint(wm.x);
             }
@@ -1706,7 +1697,7 @@ __device__ __noinline__ BigOut big_nucleus(Fin& f_in, const Filt& q_in, float y0
             census_finish(vb, t);
             if (!bit_of(e_cpl(), lb)) return out;
         }
-        if (!locate(lb, keep - 1u, e_sc()[SC_NRUNS], &run, &within)) return out;
+        if (!locate(lb, keep - 1u, &run, &within)) return out;
     }
     const uint32_t key = e_hkey()[run];
     const uint32_t minid = e_hmin()[run];
