@@ -41,6 +41,7 @@ constexpr uint32_t kHS = 2048;      // census capacity: distinct values
 constexpr uint32_t kReqMax = 512;   // bins per census
 constexpr uint32_t kReqCnt = kHS / 2;      // candidates per census (distinct values at most that many)
 constexpr uint32_t kNoBin = 0xFFFFFFFFu;
+constexpr uint32_t kNoRun = 0xFFFFFFFFu;
 constexpr uint32_t kBL = 4;         // bins per lane in a walk step
 
 // ---- LDS layout (above the re-read pass's per-tile history counts) ----------
@@ -65,7 +66,7 @@ constexpr uint32_t kOffEScd = kOffESc + 32 * 4;          // f64[8]
 constexpr uint32_t kOffEHKey = kOffEScd + 8 * 8;         // u32[kHS] census keys; runs after census_finish
 constexpr uint32_t kOffEHCnt = kOffEHKey + kHS * 4;      // u32[kHS] multiplicities
 constexpr uint32_t kOffEHMin = kOffEHCnt + kHS * 4;      // u32[kHS] smallest ids
-constexpr uint32_t kOffESort = kOffEHMin + kHS * 4;      // u64[kHS] bucket sort; then u32 run bins
+constexpr uint32_t kOffESort = kOffEHMin + kHS * 4;      // u64[kHS] bucket sort
 constexpr uint32_t kOffERunP = kOffESort + kHS * 8;      // f32[kHS] run probabilities
 constexpr uint32_t kOffEExp = kOffERunP + kHS * 4;       // u64[32] the expf table
 constexpr uint32_t kOffESHi = kOffEExp + 32 * 8;         // f32[kNB] total's value at bin starts, ties up
@@ -103,7 +104,6 @@ __device__ __forceinline__ uint32_t* e_hkey() { return e_u32(kOffEHKey); }
 __device__ __forceinline__ uint32_t* e_hcnt() { return e_u32(kOffEHCnt); }
 __device__ __forceinline__ uint32_t* e_hmin() { return e_u32(kOffEHMin); }
 __device__ __forceinline__ uint64_t* e_sort() { return reinterpret_cast<uint64_t*>(lds_base() + kOffESort); }
-__device__ __forceinline__ uint32_t* e_rbin() { return e_u32(kOffESort); }
 __device__ __forceinline__ float* e_runp() { return reinterpret_cast<float*>(lds_base() + kOffERunP); }
 __device__ __forceinline__ uint64_t* e_exptab() { return reinterpret_cast<uint64_t*>(lds_base() + kOffEExp); }
 __device__ __forceinline__ uint32_t* e_crowd() { return e_u32(kOffECrowd); }
@@ -311,7 +311,7 @@ __device__ __forceinline__ void census_take(const FBins& vb) {
 }
 
 // Turns the census into runs in list order (value descending): key,
-// multiplicity, smallest id, bin and p = exp((y - y0) / t), each bucket (one
+// multiplicity, smallest id and p = exp((y - y0) / t), each bucket (one
 // bin) ranked by comparing keys.  Returns the number of runs.
 __device__ uint32_t census_finish(const FBins& vb, float t) {
     const uint32_t tid = threadIdx.x;
@@ -337,7 +337,7 @@ __device__ uint32_t census_finish(const FBins& vb, float t) {
     TSM_LDS_SYNC();
     // e_bcnt()[i] is now the end of bucket i
     constexpr uint32_t kPer = kHS / kBlock;
-    uint32_t fin[kPer], fk[kPer], fc[kPer], fm[kPer], fb[kPer];
+    uint32_t fin[kPer], fk[kPer], fc[kPer], fm[kPer];
     float fp[kPer];
 #pragma unroll
     for (uint32_t k = 0; k < kPer; k++) {
@@ -347,8 +347,7 @@ __device__ uint32_t census_finish(const FBins& vb, float t) {
             const uint64_t me = e_sort()[pos];
             const uint32_t key = ~static_cast<uint32_t>(me >> 32), slot = static_cast<uint32_t>(me);
             const float y = key_to_float(key);
-            const uint32_t b = vb.bin(y);
-            const uint32_t ci = req_rank(b);
+            const uint32_t ci = req_rank(vb.bin(y));
             const uint32_t bs = ci ? e_bcnt()[ci - 1] : 0u, be = e_bcnt()[ci];
             uint32_t rank = 0;
             for (uint32_t j = bs; j < be; j++) rank += e_sort()[j] < me ? 1u : 0u;
@@ -356,7 +355,6 @@ __device__ uint32_t census_finish(const FBins& vb, float t) {
             fk[k] = key;
             fc[k] = e_hcnt()[slot];
             fm[k] = e_hmin()[slot];
-            fb[k] = b;
             fp[k] = glibc_expf_lds((y - vb.vb.y0) / t, e_exptab());
         }
     }
@@ -367,7 +365,6 @@ __device__ uint32_t census_finish(const FBins& vb, float t) {
             e_hkey()[fin[k]] = fk[k];
             e_hcnt()[fin[k]] = fc[k];
             e_hmin()[fin[k]] = fm[k];
-            e_rbin()[fin[k]] = fb[k];
             e_runp()[fin[k]] = fp[k];
         }
     TSM_LDS_SYNC();
@@ -440,7 +437,8 @@ struct Walk {
     float x;          // the fold's value
     uint32_t b;       // next bin
     uint32_t pos;     // candidates folded so far
-    uint32_t run;     // W_DECIDED: the deciding run and the index within it
+    uint32_t run;     // W_DECIDED (in bin b): the deciding run, kNoRun when the census has
+                      // been replaced since, and the index within it
     uint32_t within;
     uint32_t tied;    // a bound walk added a bin sum holding a tie (else its result is exact)
 };
@@ -1191,7 +1189,9 @@ __device__ __noinline__ uint32_t run_walk(Fin& f_in, const Filt& q_in, const FBi
 // lacks a bin.  The walks read the same sums and census and write their own
 // bin-start records (e_sstart, e_shi; e_pstart gets the same positions from
 // both).  Sets *rl and *rh; returns W_NEED when a bin holds more distinct
-// values than the census, else W_DONE.
+// values than the census, else W_DONE.  A census round for one walk replaces
+// the runs the other has decided by: its run is then kNoRun, and the caller
+// finds it again (locate) from its bin and position.
 constexpr uint32_t kSc2 = 16;  // e_sc() words 16..29: the two walks' results, 7 words each
 template <int K>
 __device__ __noinline__ uint32_t run_walk2(Fin& f_in, const Filt& q_in, const FBins& vb_in, Walk& wl_io,
@@ -1263,6 +1263,8 @@ __device__ __noinline__ uint32_t run_walk2(Fin& f_in, const Filt& q_in, const FB
         }
         if (n0 && w0.b == b) from0 = b;
         if (n1 && w1.b == b) from1 = b;
+        if (!n0) w0.run = kNoRun;
+        if (!n1) w1.run = kNoRun;
         census_clear();
         eng_pass<EP_CENSUS>(f, q, vb, 0.0f);
         census_finish(vb, f.m.t);
@@ -1274,8 +1276,22 @@ __device__ __noinline__ uint32_t run_walk2(Fin& f_in, const Filt& q_in, const FB
     return W_DONE;
 }
 
-// The kept candidate at position pos (0-based, pos < kept count) when no step
-// of the draw decides: its run and index within the run, from bin lb's runs.
+// Has the census hold bin b, by a round for it alone when the current one does
+// not; false when the bin holds more distinct values than the census.
+__device__ __forceinline__ bool census_bin(Fin& f, const Filt& q, const FBins& vb, uint32_t b) {
+    if (bit_of(e_cpl(), b)) return true;
+    const uint32_t tid = threadIdx.x;
+    TSM_LDS_SYNC();  // every thread has seen that the bin is missing
+    if (tid < kNB / 32u) e_req()[tid] = b / 32u == tid ? 1u << (b & 31u) : 0u;
+    TSM_LDS_SYNC();
+    census_clear();
+    eng_pass<EP_CENSUS>(f, q, vb, 0.0f);
+    census_finish(vb, f.m.t);
+    return bit_of(e_cpl(), b);
+}
+
+// The candidate at position pos (0-based) of the list, in bin lb: its run and
+// index within the run, from the bin's runs.
 __device__ __forceinline__ bool locate(uint32_t lb, uint32_t pos, uint32_t* run, uint32_t* within) {
     uint32_t r0, r1;
     runs_of(lb, &r0, &r1);
@@ -1607,7 +1623,7 @@ __device__ __noinline__ BigOut big_nucleus(Fin& f_in, const Filt& q_in, float y0
         }
         if (ra == W_DECIDED) {  // acc >= top_p at candidate wa.pos - 1 (sampler.rs:241-243)
             keep = wa.pos;
-            kb = e_rbin()[wa.run];
+            kb = wa.b;
             if (__float_as_uint(e_sstart()[kb]) != __float_as_uint(e_shi()[kb])) {
                 // total's value at bin kb still depends on a tie: total's sums
                 // again (acc's took their slots) and its exact walk
@@ -1622,17 +1638,8 @@ __device__ __noinline__ BigOut big_nucleus(Fin& f_in, const Filt& q_in, float y0
                 we.pos = e_pstart()[ba];
                 if (run_walk<FK_S>(f, q, vb, we, kb + 1u, 0.0f, 0.0f, kNoBin, 0xFFFFFFFFu, draw, false) == W_NEED)
                     return out;
-                if (!bit_of(e_cpl(), kb)) {
-                    if (tid < kNB / 32u) e_req()[tid] = 0u;
-                    TSM_LDS_SYNC();
-                    if (tid == 0) set_bit(e_req(), kb);
-                    TSM_LDS_SYNC();
-                    census_clear();
-                    eng_pass<EP_CENSUS>(f, q, vb, 0.0f);
-                    census_finish(vb, t);
-                    if (!bit_of(e_cpl(), kb)) return out;
-                }
             }
+            if (!census_bin(f, q, vb, kb)) return out;
             if (tid < kWave) {  // the kept mass: total's fold through the kept part of bin kb
                 Walk wm;
                 wm.tied = 0;
@@ -1687,17 +1694,9 @@ __device__ __noinline__ BigOut big_nucleus(Fin& f_in, const Filt& q_in, float y0
             TSM_LDS_SYNC();
             lb = e_sc()[SC_LAST];
         }
-        if (!bit_of(e_cpl(), lb)) {
-            if (tid < kNB / 32u) e_req()[tid] = 0u;
-            TSM_LDS_SYNC();
-            if (tid == 0) set_bit(e_req(), lb);
-            TSM_LDS_SYNC();
-            census_clear();
-            eng_pass<EP_CENSUS>(f, q, vb, 0.0f);
-            census_finish(vb, t);
-            if (!bit_of(e_cpl(), lb)) return out;
-        }
-        if (!locate(lb, keep - 1u, &run, &within)) return out;
+        if (!census_bin(f, q, vb, lb) || !locate(lb, keep - 1u, &run, &within)) return out;
+    } else if (run == kNoRun) {
+        if (!census_bin(f, q, vb, wr.b) || !locate(wr.b, wr.pos - 1u, &run, &within)) return out;
     }
     const uint32_t key = e_hkey()[run];
     const uint32_t minid = e_hmin()[run];
