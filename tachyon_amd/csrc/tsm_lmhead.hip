@@ -822,8 +822,10 @@ __global__ __launch_bounds__(T::kThreads) void lm_q8_gemm_line_kernel(Q8GemmArgs
 // f32 12582912 + s (|s| <= 2^19), and fma(12582912 + s, w, -12582912 w) rounds
 // s w once, as the product does; -12582912 w is exact for an f16 w.  Only the
 // sign of a zero dot's product is lost (+0 where w's sign would make -0), which
-// shows only where every term of a logit is zero: a logit that ends as +0 is
-// computed again step by step (q8_exact).
+// shows only where the exact sum is -0, that is, where every term is -0 (any
+// other partial sum is the same both ways from there on).  Such a logit ends as
+// +0 here; a workgroup that ends with +0 logits finds the -0 among them
+// (q8_zero_tile).
 //
 // A block is the 32 values of one v_mfma_i32_32x32x32_i8, so no lane group is
 // masked away.  A wave owns 64 rows x 32 JB ids (2 x JB tiles, 32 JB
@@ -837,26 +839,126 @@ constexpr uint32_t kQ8WStride = 32 * kQ8Chunk + 16;  // LDS bytes per weight row
 constexpr float kQ8Magic = 12582912.0f;
 typedef int i32x16 __attribute__((ext_vector_type(16)));
 
-// One logit as dot_q8_with adds it up.
-__device__ __noinline__ float q8_exact(const int8_t* aq, const float* as, const int8_t* w, const uint16_t* ws,
-                                       uint32_t nb) {
+// Whether a logit known to be zero is -0, adding it up as dot_q8_with does.
+__device__ __forceinline__ bool q8_negative_zero(const int8_t* aq, const float* as, const int8_t* w, const uint16_t* ws,
+                                              uint32_t nb) {
     // aq: block 0 of the row in its 16-row unit, 512 bytes a block; as: 16 floats a block
     float acc = -0.0f;
 #pragma unroll 1
-    for (uint32_t b = 0; b < nb; b++) {
+    for (uint32_t b = 0; b < nb && __float_as_uint(acc) == 0x80000000u; b++) {
         int s = 0;
 #pragma unroll 1
         for (uint32_t k = 0; k < kQ8Block; k++)
             s += static_cast<int>(aq[512u * b + 256u * (k >> 4) + (k & 15u)]) * static_cast<int>(w[kQ8Block * b + k]);
         acc = acc + static_cast<float>(s) * q8_f16(ws[b]) * as[16u * b];
     }
-    return acc;
+    return __float_as_uint(acc) == 0x80000000u;
+}
+
+// The +0 logits of a workgroup's tile (kRows x kIds from row r0, id n0) that
+// are -0.  The ids' and the rows' scales are looked through once (an id's up to
+// one above zero, which ends it for most tiles):
+//   an id with a scale above zero, a row without one so small that a product
+//   could underflow: that block's term is not -0, so +0;
+//   every dot zero (an id or a row of zeros, as padding makes them): -0 if every
+//   scale of the id has a sign, else +0;
+//   otherwise block by block until the sum is no longer -0.
+// Out of line, and the logits read back from memory, so that the multiplying
+// loop keeps its registers.  Dim 4096 by 151,936 ids, dense, a tenth of the rows
+// zero, 267 ids zero, the same under negative scales: 256 rows 541, 556, 571,
+// 610 us; 48 rows 238, 247, 241, 275 us.  (Computing every such logit again:
+// 40 to 62 ms and 12 ms.)
+struct Q8ZeroArgs {  // in LDS
+    Q8GemmArgs g;
+    uint32_t r0, n0;
+};
+enum : uint32_t { Q8_NONZERO = 1, Q8_UNSIGNED = 2, Q8_POSITIVE = 4, Q8_SMALL = 8, Q8_ASKED = 16 };
+constexpr float kQ8Small = 0x1p-100f;  // times a nonzero s w (at least 2^-24): a normal number
+
+template <uint32_t kRows, uint32_t kIds, uint32_t kThreads>
+__device__ __noinline__ void q8_zero_tile(const Q8ZeroArgs* at, uint32_t* idnote, uint32_t* rownote) {
+    const Q8GemmArgs a = at->g;
+    const uint32_t r0 = at->r0, n0 = at->n0, tid = threadIdx.x;
+    const uint32_t nb = a.dim / kQ8Block, nb2 = (nb + 1u) / 2u * 2u;
+    const uint32_t rows = min(a.rows - r0, kRows), ids = min(a.vocab - n0, kIds);
+    for (uint32_t i = tid; i < kIds; i += kThreads) idnote[i] = 0u;
+    for (uint32_t i = tid; i < kRows; i += kThreads) rownote[i] = 0u;
+    __syncthreads();
+    const uint32_t id = tid % kIds;  // this thread's id: every kThreads / kIds-th of its scales and of its logits
+    uint32_t note = 0;
+    if (id < ids) {
+        const uint16_t* sp = a.ws + static_cast<size_t>(n0 + id) * nb;
+        for (uint32_t b = tid / kIds; b < nb && !(note & Q8_POSITIVE); b += kThreads / kIds) {
+            const uint32_t h = sp[b];
+            if (h < 0x8000u) note |= h ? Q8_UNSIGNED | Q8_POSITIVE : Q8_UNSIGNED;
+        }
+        if (note) atomicOr(&idnote[id], note);
+    }
+    {
+        constexpr uint32_t kRowThreads = kThreads / (kRows / 4u);  // four rows a thread
+        const uint32_t row = 4u * (tid % (kRows / 4u)), unit = (r0 + row) >> 4;
+        note = 0;  // a byte a row
+        if (row < rows)
+#pragma unroll 16
+            for (uint32_t b = tid / (kRows / 4u); b < nb; b += kRowThreads) {
+                const f32x4 x = *reinterpret_cast<const f32x4*>(a.as + (static_cast<size_t>(unit) * nb + b) * 16u + (row & 15u));
+#pragma unroll
+                for (uint32_t e = 0; e < 4u; e++)
+                    if (x[e] != 0.0f) note |= (x[e] >= kQ8Small ? Q8_NONZERO : Q8_NONZERO | Q8_SMALL) << (8u * e);
+            }
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; e++)
+            if ((note >> (8u * e)) & 0xFFu) atomicOr(&rownote[row + e], (note >> (8u * e)) & 0xFFu);
+    }
+    const bool small = __syncthreads_or(static_cast<int>(note & (Q8_SMALL * 0x01010101u))) != 0;
+    const bool open = id < ids && (small || !(idnote[id] & Q8_POSITIVE));
+    if (!__syncthreads_or(open ? 1 : 0)) return;  // the usual end
+    uint32_t asked = 0;
+    if (open) {
+        const float* col = a.logits + static_cast<size_t>(r0) * a.ld + n0 + id;
+#pragma unroll 16
+        for (uint32_t r = tid / kIds; r < rows; r += kThreads / kIds)
+            if (__float_as_uint(col[static_cast<size_t>(r) * a.ld]) == 0u) asked = Q8_ASKED;
+        if (asked) atomicOr(&idnote[id], Q8_ASKED);
+    }
+    __syncthreads();
+    // weights, where the scales do not tell: 128 bytes a thread at a time
+    if (open && (idnote[id] & Q8_ASKED)) {
+        const int8_t* w = a.wq + static_cast<size_t>(n0 + id) * a.dim;
+        int bits = (idnote[id] & Q8_POSITIVE) ? 1 : 0;
+        for (uint32_t k0 = 128u * (tid / kIds); k0 < a.dim && !bits; k0 += 128u * (kThreads / kIds))
+#pragma unroll
+            for (uint32_t k = k0; k < k0 + 128u; k += 16u)
+                if (k < a.dim) {
+                    const i32x4 v = *reinterpret_cast<const i32x4*>(w + k);
+                    bits |= v[0] | v[1] | v[2] | v[3];
+                }
+        if (bits) atomicOr(&idnote[id], Q8_NONZERO);
+    }
+    __syncthreads();
+    if (!asked) return;
+    const uint32_t in = idnote[id];
+    for (uint32_t r = tid / kIds; r < rows; r += kThreads / kIds) {
+        const uint32_t rn = rownote[r];
+        if ((in & Q8_POSITIVE) && !(rn & Q8_SMALL)) continue;
+        float* out = a.logits + static_cast<size_t>(r0 + r) * a.ld + n0 + id;
+        if (__float_as_uint(*out) != 0u) continue;
+        const uint32_t row = r0 + r;
+        const bool neg = (in & rn & Q8_NONZERO)
+                             ? q8_negative_zero(a.aq + static_cast<size_t>(row >> 4) * nb2 * 512u + (row & 15u) * 16u,
+                                                a.as + static_cast<size_t>(row >> 4) * nb * 16u + (row & 15u),
+                                                a.wq + static_cast<size_t>(n0 + id) * a.dim,
+                                                a.ws + static_cast<size_t>(n0 + id) * nb, nb)
+                             : !(in & Q8_UNSIGNED);
+        if (neg) *out = -0.0f;
+    }
 }
 
 // kWide: nb a multiple of 4 and wscale 8-byte aligned (a chunk's scales of an
 // id are one 8-byte load; otherwise four 2-byte loads).
+// Three waves a SIMD where the tile's registers allow it (WR = 2: 161 and 168).
 template <uint32_t JB, uint32_t WR, uint32_t WN, bool kWide>
-__global__ __launch_bounds__(64 * WR * WN, 2) void lm_q8_gemm32_kernel(Q8GemmArgs a) {
+__global__ __launch_bounds__(64 * WR * WN, WR == 2u ? 3 : 2) void lm_q8_gemm32_kernel(Q8GemmArgs a) {
     constexpr uint32_t kThreads = 64u * WR * WN, kRows = 64u * WR, kIds = 32u * JB * WN;
     constexpr uint32_t kWLoads = kIds * 2u * kQ8Chunk / kThreads;  // 16-byte weight loads per thread and chunk
     constexpr uint32_t kXLoads = kRows * kQ8Chunk / 4u;            // 16-byte row scale loads per chunk
@@ -988,6 +1090,7 @@ __global__ __launch_bounds__(64 * WR * WN, 2) void lm_q8_gemm32_kernel(Q8GemmArg
         }
         __syncthreads();
     }
+    int zeros = 0;
 #pragma unroll
     for (uint32_t i = 0; i < 2u; i++)
 #pragma unroll
@@ -1000,14 +1103,18 @@ __global__ __launch_bounds__(64 * WR * WN, 2) void lm_q8_gemm32_kernel(Q8GemmArg
                 for (uint32_t j = 0; j < JB; j++) {
                     const uint32_t id = n0 + 32u * JB * wn + 32u * j + (lane & 31u);
                     if (id >= a.vocab) continue;
-                    float v = acc[i][j][g][e];
-                    if (__float_as_uint(v) == 0u)
-                        v = q8_exact(a.aq + static_cast<size_t>(row >> 4) * nb2 * 512u + (row & 15u) * 16u,
-                                     a.as + static_cast<size_t>(row >> 4) * nb * 16u + (row & 15u),
-                                     a.wq + static_cast<size_t>(id) * a.dim, a.ws + static_cast<size_t>(id) * nb, nb);
+                    const float v = acc[i][j][g][e];
+                    zeros |= __float_as_uint(v) == 0u ? 1 : 0;
                     a.logits[static_cast<size_t>(row) * a.ld + id] = v;
                 }
             }
+    if (!__syncthreads_or(zeros)) return;
+    // the stage is free now: the notes, and the arguments
+    static_assert(sizeof(Q8ZeroArgs) <= sizeof(sbuf) && kIds * 4u <= sizeof(wbuf) && kRows * 4u <= sizeof(xbuf), "fits");
+    Q8ZeroArgs* z = reinterpret_cast<Q8ZeroArgs*>(&sbuf);
+    if (tid == 0) *z = Q8ZeroArgs{a, r0, n0};
+    __syncthreads();
+    q8_zero_tile<kRows, kIds, kThreads>(z, reinterpret_cast<uint32_t*>(&wbuf), reinterpret_cast<uint32_t*>(&xbuf));
 }
 
 template <uint32_t JB, uint32_t WR, uint32_t WN>
