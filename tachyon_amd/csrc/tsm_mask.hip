@@ -708,7 +708,9 @@ int tsm_json_masks_fill(tsm_json_masks* m, void* stream, const tsm_vocab* vocab,
         const dim3 grid((m->nwords + tsm::mask::kCopyWords - 1) / tsm::mask::kCopyWords, copies + (jobs ? 1u : 0u));
         hipLaunchKernelGGL(tsm::mask::mask_copy_kernel, grid, dim3(tsm::mask::kCB), 0, s, c);
     }
-    if (jobs > 0) {
+    hipError_t e = hipGetLastError();
+    // (a failed copy brought no states: the evaluation would read what the last call left)
+    if (e == hipSuccess && jobs > 0) {
         const tsm::mask::Stage ls = tsm::mask::stage_at(m->local, m->max_rows, jobs, groups, outs);
         tsm::mask::JsonMaskArgs a;
         a.bytes = vocab->bytes;
@@ -729,10 +731,13 @@ int tsm_json_masks_fill(tsm_json_masks* m, void* stream, const tsm_vocab* vocab,
         a.per_group = per;
         hipLaunchKernelGGL((tsm::mask::json_mask_kernel<true>), dim3(blocks, groups), dim3(tsm::mask::kMB), 0, s, a);
     }
-    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipGetLastError();
     if (e == hipSuccess) e = hipEventRecord(m->used[h], s);
     if (e == hipSuccess) e = hipEventRecord(m->done, s);
-    if (e != hipSuccess) return set_err(err, errlen, "launch failed: %s", hipGetErrorString(e)), 1;
+    if (e != hipSuccess) {
+        m->flush();  // the index names the call's new states already, whose masks may never be written
+        return set_err(err, errlen, "launch failed: %s", hipGetErrorString(e)), 1;
+    }
     m->pending[h] = true;
     m->called = true;
     if (stats) {

@@ -1,0 +1,94 @@
+// tsm_json_masks_fill on the CPU emulation (test infrastructure) with launches
+// counted and made to fail: a call that failed leaves no state behind that the
+// set would take for a kept mask.  Prints "ok" and exits 0 when all holds.
+#include <hip/hip_runtime.h>
+
+#include <cstdio>
+#include <cstring>
+#include <string>
+#include <vector>
+
+static int launches = 0, fail_launch = 0, fail_record = 0, records = 0;  // fail_*: the n-th of the call, 0 none
+static hipError_t last = hipSuccess;
+template <class F>
+static void launch(F&& f) {
+    if (++launches == fail_launch) last = hipErrorInvalidValue;
+    else f();
+}
+static hipError_t last_error() {
+    const hipError_t e = last;
+    last = hipSuccess;
+    return e;
+}
+static hipError_t record(hipEvent_t e, hipStream_t s) { return ++records == fail_record ? hipErrorInvalidValue : hipEventRecord(e, s); }
+#define hipLaunchKernelGGL(...) launch([&] { hipLaunchKernelGGL(__VA_ARGS__); })
+#define hipGetLastError last_error
+#define hipEventRecord record
+#include "../../tachyon_amd/csrc/tsm_mask.hip"
+
+static int fails = 0;
+#define CHECK(c, ...)                          \
+    do {                                       \
+        if (!(c)) {                            \
+            std::fprintf(stderr, __VA_ARGS__); \
+            std::fprintf(stderr, "\n");        \
+            fails++;                           \
+        }                                      \
+    } while (0)
+
+static tsm_json_state state_of(const char* prefix) {
+    tsm_json_state s;
+    tsm_json_init(&s);
+    tsm_json_advance(&s, reinterpret_cast<const uint8_t*>(prefix), std::strlen(prefix));
+    return s;
+}
+
+int main() {
+    std::vector<uint8_t> bytes;
+    std::vector<uint32_t> offsets{0}, special(10, 0u);
+    for (uint32_t t = 0; t < 300; t++) {
+        bytes.push_back(static_cast<uint8_t>(t));
+        if (t >= 256) bytes.push_back(static_cast<uint8_t>("\"}],:0e {"[t % 9]));
+        offsets.push_back(static_cast<uint32_t>(bytes.size()));
+    }
+    const tsm_vocab v{bytes.data(), offsets.data(), special.data(), 300, 0};
+    const uint32_t usable = 300, nw = (usable + 31) / 32;
+    const std::vector<tsm_json_state> a = {state_of("{"), state_of("{\"a\":"), state_of("{"), state_of("{\"k")};
+    const std::vector<tsm_json_state> b = {state_of("{\"x\": 1"), state_of("{\"k"), state_of("{\"y\": [")};
+    char err[128];
+    // a call's results, or a failed one's code; counts what it launched
+    auto fill = [&](tsm_json_masks* m, const std::vector<tsm_json_state>& rows, tsm_json_fill_stats* st) {
+        std::vector<uint32_t> got(rows.size() * nw, 0x5A5A5A5Au), want(rows.size() * nw, 0u);
+        launches = records = 0;
+        const int rc = tsm_json_masks_fill(m, nullptr, &v, rows.data(), static_cast<uint32_t>(rows.size()), got.data(), nw,
+                                           st, err, sizeof(err));
+        fail_launch = fail_record = 0;
+        if (rc != 0) return rc;
+        for (size_t r = 0; r < rows.size(); r++)
+            for (uint32_t t = 0; t < usable; t++)
+                if (tsm_json_accepts(&rows[r], bytes.data() + offsets[t], offsets[t + 1] - offsets[t]))
+                    want[r * nw + t / 32] |= 1u << (t % 32);
+        CHECK(got == want, "a call's masks differ from the host automaton's");
+        return rc;
+    };
+    // the n-th launch, and each event record, fails: with an empty set, and with one that holds some of the rows
+    for (int kept = 0; kept < 2; kept++)
+        for (int n = 1; n <= 4; n++) {
+            tsm_json_masks* m = tsm_json_masks_create(0, 8, 8, usable, err, sizeof(err));
+            tsm_json_fill_stats st;
+            if (kept) CHECK(fill(m, b, &st) == 0, "fill: %s", err);
+            (n <= 2 ? fail_launch : fail_record) = n <= 2 ? n : n - 2;
+            const int rc = fill(m, a, &st);
+            if (n > 2 || launches >= n) {  // a call of one launch has no second one to fail
+                CHECK(rc != 0, "kept %d, failure %d: reported as done", kept, n);
+                CHECK(n != 1 || launches == 1, "kept %d: %d launches after the first failed", kept, launches);
+                CHECK(fill(m, a, &st) == 0, "fill after a failure: %s", err);
+                CHECK(st.hits == 0 && st.evaluated == 3, "kept %d, failure %d: %u hits, %u evaluated after it", kept, n,
+                      st.hits, st.evaluated);
+            }
+            tsm_json_masks_destroy(m);
+        }
+    if (fails) return 1;
+    std::printf("ok\n");
+    return 0;
+}
