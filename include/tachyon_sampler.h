@@ -306,8 +306,8 @@ int tsm_json_mask(void* stream, const tsm_vocab* vocab, const tsm_json_state* st
  * tsm_json_masks_fill: `states` is a HOST array of `rows` (<= max_rows)
  * states, as tsm_json_advance keeps them; `mask` (device) gets one row per
  * state, words [0, ceil(usable / 32)) of each written.  `stats` (may be NULL)
- * receives the call's counts.  Queued on `stream`: one copy launch and at
- * most one evaluation launch.  The call waits on the host only for the
+ * receives the call's counts.  Queued on `stream`: at most one copy launch
+ * and one evaluation launch.  The call waits on the host only for the
  * launches of the call before the last one (the staging alternates between
  * two halves).  The slots are tied to the
  * vocabulary's device pointers and n_tokens: a call with other ones empties

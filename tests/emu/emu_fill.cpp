@@ -1,6 +1,7 @@
 // tsm_json_masks_fill on the CPU emulation (test infrastructure) with launches
 // counted and made to fail: a call that failed leaves no state behind that the
-// set would take for a kept mask.  Prints "ok" and exits 0 when all holds.
+// set would take for a kept mask, and a call that copies no row makes one
+// launch.  Prints "ok" and exits 0 when all holds.
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
@@ -88,6 +89,17 @@ int main() {
             }
             tsm_json_masks_destroy(m);
         }
+    {  // one launch where no row is copied: rows in new states, or a set keeping nothing
+        tsm_json_masks* m = tsm_json_masks_create(0, 8, 8, usable, err, sizeof(err));
+        tsm_json_masks* m0 = tsm_json_masks_create(0, 8, 0, usable, err, sizeof(err));
+        tsm_json_fill_stats st;
+        CHECK(fill(m, {a[0]}, &st) == 0 && launches == 1, "a new state: %d launches", launches);
+        CHECK(fill(m, {a[0]}, &st) == 0 && launches == 1, "a kept state: %d launches", launches);
+        CHECK(fill(m, a, &st) == 0 && launches == 2, "kept and new states: %d launches", launches);
+        CHECK(fill(m0, a, &st) == 0 && launches == 1, "nothing kept: %d launches", launches);
+        tsm_json_masks_destroy(m);
+        tsm_json_masks_destroy(m0);
+    }
     if (fails) return 1;
     std::printf("ok\n");
     return 0;
