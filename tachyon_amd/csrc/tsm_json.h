@@ -295,13 +295,15 @@ enum : uint32_t {
     W_END = 1u << 15,      // a value ended: what follows depends on the depth
     W_COMMA = 1u << 16,    // what follows depends on the container
     W_REJECT = 1u << 17,
-    W_RESET = 18
+    W_RESET = 18,
+    W_TEXT = 1u << 23      // string text follows: a rest of text bytes only passes whole
 };
 struct Entry {
     uint32_t x, y;
 };
 constexpr Entry entry(uint32_t flat, uint32_t flags, uint32_t add = 0, uint32_t reset = 0) {
-    return Entry{flat * kClasses | flags | reset << W_RESET, add};
+    const bool text = flat == F_STR || flat == F_STR + 6u;
+    return Entry{flat * kClasses | flags | (text ? uint32_t(W_TEXT) : 0u) | reset << W_RESET, add};
 }
 // the steps a byte can make
 constexpr Entry e_reject(uint32_t f) { return entry(f, W_REJECT | W_USED); }

@@ -57,6 +57,7 @@ constexpr uint32_t kWords = kTok / 32;
 constexpr uint32_t kQueue = 128;     // a wave's open (state, token) pairs: settled above 64, 64 more at a time
 constexpr int kTakeAt = 24;          // free lanes that make a wave take new pairs
 constexpr uint32_t kToSlot = 0x80000000u;
+constexpr uint32_t kPlain = 0x80000000u;  // a token of text bytes only
 constexpr uint32_t kText = 0x80000000u;   // inside a string, no escape pending
 constexpr uint32_t kOther = 0x80000000u;  // the first classes of a state the tables do not hold
 
@@ -123,9 +124,9 @@ __global__ __launch_bounds__(kMB) void json_mask_kernel(JsonMaskArgs a) {
     __shared__ uint32_t table[kHashed];
     __shared__ uint32_t wave_n[kStates / kWave];
     __shared__ uint32_t bits[kStates * kWords];
-    __shared__ uint32_t tok_off[kTok];                // stage offset | length << 16
+    __shared__ uint32_t tok_off[kTok];                // stage offset | length << 16 | kPlain
     __shared__ uint16_t queue[kWaves][kQueue];
-    static_assert(kStage <= 65536u && kStates * kWave <= 65536u, "16-bit offsets and queue entries");
+    static_assert(kStage <= 32768u && kStates * kWave <= 65536u, "16-bit offsets and queue entries, a bit beside a length");
     const uint32_t tid = threadIdx.x, lane = lane_id(), wid = tid / kWave;
     const uint32_t t0 = blockIdx.x * kTok;
     const uint32_t lim = a.usable < a.n_tokens ? a.usable : a.n_tokens;  // ids with bytes that count
@@ -215,7 +216,7 @@ __global__ __launch_bounds__(kMB) void json_mask_kernel(JsonMaskArgs a) {
                 odd |= w;
             }
             plain = (odd & (json::kNotText * 0x01010101u)) == 0u;
-            if (wid % kSplit == 0) tok_off[tt] = (b0 - lo) | (b1 - b0) << 16;
+            if (wid % kSplit == 0) tok_off[tt] = (b0 - lo) | (b1 - b0) << 16 | (plain ? kPlain : 0u);
         } else {
             if (has) c1 = cls[a.bytes[b0]] & (json::kClasses - 1u);
             if (wid % kSplit == 0) tok_off[tt] = 0u;  // no length: stepped from global memory
@@ -223,9 +224,9 @@ __global__ __launch_bounds__(kMB) void json_mask_kernel(JsonMaskArgs a) {
     }
     __syncthreads();
     // the pair this lane walks: its automaton, the classes still to come (none
-    // left: the lane is free) and where its answer goes
+    // left: the lane is free), whether its token is plain and where its answer goes
     json::Walk walk = {0u, 0u, 0u};
-    uint32_t from = 0, to = 0, answer = 0;
+    uint32_t from = 0, to = 0, text = 0, answer = 0;
     uint32_t open = 0;  // pairs in the queue (wave-uniform)
     // free lanes take the queue's last pairs (state q >> 6, this wave's token q & 63)
     auto take = [&](uint64_t free) {
@@ -236,7 +237,8 @@ __global__ __launch_bounds__(kMB) void json_mask_kernel(JsonMaskArgs a) {
             walk = walks[s];
             const uint32_t ol = tok_off[t];
             from = ol & 0xFFFFu;
-            to = from + (ol >> 16);
+            to = from + ((ol & ~kPlain) >> 16);
+            text = (ol & kPlain) ? uint32_t(json::W_TEXT) : 0u;
             answer = s * kTok + t;
         }
         const uint32_t n = static_cast<uint32_t>(__popcll(free));
@@ -257,8 +259,11 @@ __global__ __launch_bounds__(kMB) void json_mask_kernel(JsonMaskArgs a) {
                 const json::Entry e = next[walk.row + (stage[from] & (json::kClasses - 1u))];
                 const bool ok = json::step_entry(walk, e);
                 from += (e.x / json::W_USED) & 1u;
-                if (!ok) from = to;
-                else if (from == to) atomicOr(&bits[answer >> 5], 1u << (answer & 31u));
+                // a plain token that has come to a string's text (after an escape,
+                // say) passes: stepped to its end, 16 rows of 16,000 ids with a
+                // 63-byte token took 20 us, the walk in place before 17
+                if (!ok || (e.x & text)) from = to;
+                if (ok && from == to) atomicOr(&bits[answer >> 5], 1u << (answer & 31u));
             }
         }
         wave_lds_order();

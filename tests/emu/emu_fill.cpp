@@ -50,6 +50,11 @@ int main() {
     for (uint32_t t = 0; t < 300; t++) {
         bytes.push_back(static_cast<uint8_t>(t));
         if (t >= 256) bytes.push_back(static_cast<uint8_t>("\"}],:0e {"[t % 9]));
+        if (t >= 270) {  // tokens of text bytes only, or but for their last byte
+            const std::string tail = std::string("u00e9bnf/rt00ab") + std::string(t % 40, 'x') + (t % 3 ? "" : "\"");
+            bytes.resize(offsets.back());
+            bytes.insert(bytes.end(), tail.begin() + t % 15, tail.end());
+        }
         offsets.push_back(static_cast<uint32_t>(bytes.size()));
     }
     const tsm_vocab v{bytes.data(), offsets.data(), special.data(), 300, 0};
@@ -99,6 +104,16 @@ int main() {
         CHECK(fill(m0, a, &st) == 0 && launches == 1, "nothing kept: %d launches", launches);
         tsm_json_masks_destroy(m);
         tsm_json_masks_destroy(m0);
+    }
+    {  // states inside strings, escapes and \\u groups among them, which plain tokens leave for text
+        std::vector<tsm_json_state> in;
+        for (const char* p : {"{\"a", "{\"a\\", "{\"a\\u", "{\"a\\u0", "{\"a\\u00", "{\"a\\u00e", "{\"a\": \"\\", "[\"\\u12",
+                              "{\"a\": [\"b\\u", "{\"a\": 1", "{\"a\": tr"})
+            in.push_back(state_of(p));
+        tsm_json_masks* m = tsm_json_masks_create(0, 16, 0, usable, err, sizeof(err));
+        tsm_json_fill_stats st;
+        CHECK(fill(m, in, &st) == 0, "fill: %s", err);
+        tsm_json_masks_destroy(m);
     }
     if (fails) return 1;
     std::printf("ok\n");
