@@ -48,9 +48,12 @@ constexpr uint32_t kSplit = 2;       // waves that share 64 tokens, each with it
 constexpr int kMB = static_cast<int>(kTok * kSplit);  // threads per workgroup
 constexpr uint32_t kStates = 256;    // states per workgroup at most
 constexpr uint32_t kHashed = 2 * kStates;  // slots of the table that finds equal states
-// Workgroups a launch aims for: a short vocabulary's states go to several
-// groups.  Above the token blocks' own number a full vocabulary's states would
-// be split too, and equal ones no longer meet (1024: 63 us against 45).
+// Workgroups a launch aims for, two a CU: a short vocabulary's states go to
+// several groups, as many as come nearest to it.  Split states pay the fixed
+// part twice and equal ones no longer meet, so a vocabulary of 342 blocks on
+// stays whole: 256 rows, one group against two, 151,936 ids (594 blocks) 45
+// against 63 us (before plain tokens passed at once), 128,256 (501) 30.7
+// against 38.2, 100,352 (392) 30.5 against 37.0, 80,000 (313) 29.9 against 28.5.
 constexpr uint32_t kFillGroups = 512;
 constexpr uint32_t kStage = 16384;   // LDS bytes for the workgroup's tokens
 constexpr uint32_t kWords = kTok / 32;
@@ -82,10 +85,11 @@ struct JsonMaskArgs {
 };
 
 // States per workgroup for `n` states over `blocks` token blocks: all of them
-// (so that equal ones meet) up to kStates, fewer while that leaves the launch
-// below kFillGroups workgroups.
+// (so that equal ones meet) up to kStates, or split into as many groups as
+// bring the launch nearest to kFillGroups workgroups.
 inline uint32_t states_per_group(uint32_t n, uint32_t blocks) {
-    const uint32_t want_y = (kFillGroups + blocks - 1) / blocks;
+    const uint32_t near = (kFillGroups + blocks / 2u) / blocks;
+    const uint32_t want_y = near > 1u ? near : 1u;
     const uint32_t gy = want_y < n ? want_y : n;
     const uint32_t per = (n + gy - 1) / gy;
     return per < kStates ? per : kStates;

@@ -1,7 +1,7 @@
 // tsm_json_masks_fill on the CPU emulation (test infrastructure) with launches
 // counted and made to fail: a call that failed leaves no state behind that the
 // set would take for a kept mask, and a call that copies no row makes one
-// launch.  Prints "ok" and exits 0 when all holds.
+// launch, its states grouped by the vocabulary's length.  Prints "ok" and exits 0 when all holds.
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
@@ -114,6 +114,15 @@ int main() {
         tsm_json_fill_stats st;
         CHECK(fill(m, in, &st) == 0, "fill: %s", err);
         tsm_json_masks_destroy(m);
+    }
+    {  // a full vocabulary's states stay together, so that equal ones meet; a short one's are spread
+        using tsm::mask::states_per_group;
+        for (uint32_t blocks : {392u, 501u, 594u, 1024u})
+            CHECK(states_per_group(256, blocks) == 256 && states_per_group(700, blocks) == 256 && states_per_group(1, blocks) == 1,
+                  "%u blocks: %u states a group", blocks, states_per_group(256, blocks));
+        CHECK(states_per_group(256, 313) == 128 && states_per_group(256, 125) == 64 && states_per_group(16, 1) == 1,
+              "short vocabularies: %u %u %u states a group", states_per_group(256, 313), states_per_group(256, 125),
+              states_per_group(16, 1));
     }
     if (fails) return 1;
     std::printf("ok\n");
