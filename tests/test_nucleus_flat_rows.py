@@ -38,8 +38,11 @@ def test_decided_walk_survives_a_census_round_on_the_cpu_emulation(case):
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", ROWS)
 def test_decided_walk_survives_a_census_round_on_the_gpu(case):
+    import torch
+
     from tachyon_amd.device import SamplerContext, run_workload
 
+    torch.cuda.init()  # before the library's first call
     w = flat_row(*case)
     ctx = SamplerContext(max_rows=1, max_vocab=USABLE)
     try:
