@@ -125,7 +125,6 @@ enum : uint32_t {  // e_sc() words
     SC_X = 11,
     SC_OVF = 12,    // census table full
     SC_CMIN = 13,   // smallest candidate value's total key
-    SC_TIED = 14,   // walk: a bin sum it added holds a tie
     SC_FILED = 15,  // elements filed for the census
 };
 
@@ -178,14 +177,12 @@ __device__ __forceinline__ int step_binade(float x, bool sub) {
 
 constexpr uint32_t kTieTerm = 0xFFFFFFFFu;  // tau halfway between grid points
 constexpr uint32_t kBigTerm = 0xFFFFFFFEu;  // tau >= 2^(e+1): no grid sum holds its step
-// RN_e(tau) in grid units of binade e, or kTieTerm (tau exactly halfway
-// between grid points; *fl gets the lower one) or kBigTerm.
-__device__ __forceinline__ uint32_t grid_term(float tau, int e, uint32_t* fl = nullptr) {
+// RN_e(tau) in grid units of binade e, or kTieTerm or kBigTerm.
+__device__ __forceinline__ uint32_t grid_term(float tau, int e) {
     if (!(tau < ldexpf(1.0f, e + 1))) return kBigTerm;
     const float v = ldexpf(tau, -grid_of(e));  // < 2^24: exact
     const float k = floorf(v);
     const float fr = v - k;
-    if (fl) *fl = static_cast<uint32_t>(k);
     if (fr == 0.5f) return kTieTerm;
     return static_cast<uint32_t>(k) + (fr > 0.5f ? 1u : 0u);
 }
@@ -312,8 +309,8 @@ __device__ __forceinline__ void census_take(const FBins& vb) {
 
 // Turns the census into runs in list order (value descending): key,
 // multiplicity, smallest id and p = exp((y - y0) / t), each bucket (one
-// bin) ranked by comparing keys.  Returns the number of runs.
-__device__ uint32_t census_finish(const FBins& vb, float t) {
+// bin) ranked by comparing keys.
+__device__ void census_finish(const FBins& vb, float t) {
     const uint32_t tid = threadIdx.x;
     for (uint32_t i = tid; i < kReqMax; i += kBlock) e_bcnt()[i] = 0u;
     TSM_LDS_SYNC();
@@ -368,7 +365,6 @@ __device__ uint32_t census_finish(const FBins& vb, float t) {
             e_runp()[fin[k]] = fp[k];
         }
     TSM_LDS_SYNC();
-    return total;
 }
 
 // First run of a censused bin b and the end of its runs: census_finish leaves
@@ -440,7 +436,6 @@ struct Walk {
     uint32_t run;     // W_DECIDED (in bin b): the deciding run, kNoRun when the census has
                       // been replaced since, and the index within it
     uint32_t within;
-    uint32_t tied;    // a bound walk added a bin sum holding a tie (else its result is exact)
 };
 
 // The runs [r0, r1) of one bin, in order, folding at most up to candidate
@@ -553,7 +548,7 @@ __device__ uint32_t walk_bins(Walk& w, uint32_t bend, float T, float thr, uint32
             const uint32_t bl = w.b + kBL * lane;
             uint32_t nj[kBL], cj[kBL];
             bool okj[kBL];
-            uint32_t ln = 0, lc = 0, tmask = 0;  // tmask: the lane's summable bins holding a tie
+            uint32_t ln = 0, lc = 0;
             // every word of the lane's bins first, whatever the plans turn out
             // to say: one wait for LDS instead of one a bin and condition (with
             // the runs found by their bucket: 60 -> 40 us for total's two walks
@@ -585,7 +580,6 @@ __device__ uint32_t walk_bins(Walk& w, uint32_t bend, float T, float thr, uint32
                 bool ok = (low || high) && b != force && (kB == 0 ? !tie : !bad);
                 uint32_t c = min(high ? s1[j] : s0[j], 1u << 25) + (kB == 2 && tie ? 1u : 0u);
                 const bool take = ok && n != 0u;
-                if (kB != 0 && take && tie) tmask |= 1u << j;
                 c = take ? c : 0u;
                 ok = b < bend && (ok || n == 0u);  // past bend: the end marker; an empty bin passes
                 // past 2^25 units a bin leaves the binade anyway: the clamps keep
@@ -635,10 +629,6 @@ __device__ uint32_t walk_bins(Walk& w, uint32_t bend, float T, float thr, uint32
                 np += nj[j];
             }
             const uint32_t f = first_lane(wave_ballot(jb < kBL));
-            if (kB != 0) {  // the bins added below: every bin of the lanes before f, lane f's before jb
-                const uint32_t applied = lane < f ? tmask : (lane == f ? tmask & ((1u << jb) - 1u) : 0u);
-                if (wave_ballot(applied != 0u)) w.tied = 1u;
-            }
             // lanes after f recorded bin starts past the stop; the next step
             // writes them again from the right value
             if (f == 64u) {
@@ -708,8 +698,10 @@ __device__ __forceinline__ void add_term(uint32_t slot, uint32_t b, float tau, i
 // relative error is below 2^-51, and no quotient of two f32 values lies within
 // 2^-49 of the middle between two f32 values (its distance from one is a
 // nonzero multiple of 2^-24 / b in units of the middle's last place), so it
-// rounds as the quotient does.  (A subnormal quotient may round otherwise: exp
-// of it is 1 either way.)  A third of the instructions of the f32 division.
+// rounds as the quotient does.  A subnormal quotient may round otherwise, which
+// shows nowhere: exp of (y - y0) / t is 1 then, and a p / total that small is
+// none of acc's grid units, whose first term is 1 / total.  A third of the
+// instructions of the f32 division.
 __device__ __forceinline__ float quotient(float a, double inv) {
     return static_cast<float>(static_cast<double>(a) * inv);
 }
@@ -1193,7 +1185,6 @@ __device__ __noinline__ uint32_t run_walk(Fin& f_in, const Filt& q_in, const FBi
                 e_sc()[SC_RUN] = w.run;
                 e_sc()[SC_WITHIN] = w.within;
                 e_sc()[SC_X] = __float_as_uint(w.x);
-                e_sc()[SC_TIED] = w.tied;
             }
         }
         TSM_LDS_SYNC();
@@ -1203,7 +1194,6 @@ __device__ __noinline__ uint32_t run_walk(Fin& f_in, const Filt& q_in, const FBi
         w.run = e_sc()[SC_RUN];
         w.within = e_sc()[SC_WITHIN];
         w.x = __uint_as_float(e_sc()[SC_X]);
-        w.tied = e_sc()[SC_TIED];
         TSM_LDS_SYNC();
         if (res != W_NEED) {
             w_io = w;
@@ -1242,7 +1232,7 @@ __device__ __noinline__ uint32_t run_walk(Fin& f_in, const Filt& q_in, const FBi
 // values than the census, else W_DONE.  A census round for one walk replaces
 // the runs the other has decided by: its run is then kNoRun, and the caller
 // finds it again (locate) from its bin and position.
-constexpr uint32_t kSc2 = 16;  // e_sc() words 16..29: the two walks' results, 7 words each
+constexpr uint32_t kSc2 = 16;  // e_sc() words 16..27: the two walks' results, 6 words each
 template <int K>
 __device__ __noinline__ uint32_t run_walk2(Fin& f_in, const Filt& q_in, const FBins& vb_in, Walk& wl_io,
                                            Walk& wh_io, uint32_t* rl, uint32_t* rh, uint32_t bend, float T,
@@ -1261,28 +1251,26 @@ __device__ __noinline__ uint32_t run_walk2(Fin& f_in, const Filt& q_in, const FB
             const uint32_t res = wid == 0u ? walk_bins<K, 1>(w, bend, T, thr, force, lim)
                                            : walk_bins<K, 2>(w, bend, T, thr, force, lim);
             if (lane_id() == 0) {
-                uint32_t* o = e_sc() + kSc2 + 7u * wid;
+                uint32_t* o = e_sc() + kSc2 + 6u * wid;
                 o[0] = res;
                 o[1] = w.b;
                 o[2] = w.pos;
                 o[3] = w.run;
                 o[4] = w.within;
                 o[5] = __float_as_uint(w.x);
-                o[6] = w.tied;
             }
         }
         TSM_LDS_SYNC();
 #pragma unroll
         for (uint32_t j = 0; j < 2u; j++) {
             if ((j == 0u ? r0 : r1) != W_NEED) continue;
-            const uint32_t* o = e_sc() + kSc2 + 7u * j;
+            const uint32_t* o = e_sc() + kSc2 + 6u * j;
             Walk& w = j == 0u ? w0 : w1;
             w.b = o[1];
             w.pos = o[2];
             w.run = o[3];
             w.within = o[4];
             w.x = __uint_as_float(o[5]);
-            w.tied = o[6];
             if (j == 0u) r0 = o[0];
             else r1 = o[0];
         }
@@ -1631,7 +1619,7 @@ __device__ __noinline__ BigOut big_nucleus(Fin& f_in, const Filt& q_in, float y0
     w0.x = 0.0f;
     w0.b = 0;
     w0.pos = 0;
-    w0.run = w0.within = w0.tied = 0;
+    w0.run = w0.within = 0;
     // total: with every unresolved tie rounded down, then up; when both give
     // the same value it is total (the fold is monotone in each step), else
     // the ties are censused and stepped exactly
@@ -1696,7 +1684,6 @@ __device__ __noinline__ BigOut big_nucleus(Fin& f_in, const Filt& q_in, float y0
             if (!census_bin(f, q, vb, kb)) return out;
             if (tid < kWave) {  // the kept mass: total's fold through the kept part of bin kb
                 Walk wm;
-                wm.tied = 0;
                 wm.x = e_sstart()[kb];
                 wm.b = kb;
                 wm.pos = e_pstart()[kb];
@@ -1721,7 +1708,7 @@ __device__ __noinline__ BigOut big_nucleus(Fin& f_in, const Filt& q_in, float y0
     wr.x = u * mass;
     wr.b = 0;
     wr.pos = 0;
-    wr.run = wr.within = wr.tied = 0;
+    wr.run = wr.within = 0;
     const uint32_t bend = kb != kNoBin ? kb + 1u : kNB;
     // the draw with unresolved ties one way and the other at once; the same pick
     // from both is the draw's, else the exact walk
