@@ -291,8 +291,9 @@ int tsm_json_mask(void* stream, const tsm_vocab* vocab, const tsm_json_state* st
  * (every row writing string text at one depth, say) and states recur from step
  * to step.  Each call evaluates every distinct state of its rows once, keeps
  * the masks of up to `capacity` states in device memory (least recently used
- * out first), and fills each row's mask by a copy from its state's mask.  The
- * masks written are the ones tsm_json_mask writes for the same states.
+ * out first), and fills each row's mask: a kept state's by a copy, a new
+ * state's as it is evaluated.  The masks written are the ones tsm_json_mask
+ * writes for the same states.
  * Replaces: the same closure as tsm_json_mask (src/scheduler.rs:653-656),
  * with the per-state reuse the reference's probing has no need of.
  *

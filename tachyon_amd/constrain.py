@@ -106,7 +106,7 @@ def json_mask(vocab: DeviceVocab, states_dev, rows: int, usable: int, mask_dev, 
 class JsonMaskSet:
     """tsm_json_masks_*: masks of recent JsonObject states kept on the GPU;
     each fill evaluates every distinct state of its rows once (reusing the
-    kept ones) and copies each row's mask from its state's."""
+    kept ones), whose rows are written with it; the others' masks are copied."""
 
     def __init__(self, max_rows: int, capacity: int, usable: int, device: int = 0):
         err = _lib._err()

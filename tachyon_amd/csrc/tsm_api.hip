@@ -248,7 +248,8 @@ static int queue(hipStream_t s, const tsm_batch* b, const tsm_outputs* out, uint
     // workgroup per row would leave most of the chip idle; from
     // kSplitRowsMax rows on, the whole-row kernels sample every row.  The
     // lean kernel takes the common top-k rows, the general kernel every
-    // other; distribution() always takes the general kernel.
+    // other.  distribution()'s split-kind rows go to the split kernel too; its
+    // other rows always to the general kernel.
     uint32_t kinds = b->row_kinds ? b->row_kinds : (TSM_ROWKIND_SPLIT | TSM_ROWKIND_WHOLE | TSM_ROWKIND_LEAN);
     if (b->rows > tsm::split::kSplitRowsMax || !split) {
         // a split-kind row takes a whole-row kernel: the one its kind names

@@ -9,7 +9,8 @@
 // with one ballot; the (state, token) pairs still open go to a queue of the
 // wave's own and are stepped 64 at a time, one pair a lane, through the
 // automaton's table (tsm_json.h), so that no lane waits for a neighbour whose
-// token was decided at once.  The answers are collected in LDS, a word per
+// token was decided at once; a plain token passes as soon as its walk comes to
+// a string's text.  The answers are collected in LDS, a word per
 // state and 32 tokens, and written to every row of the state at the end.
 //
 // What bounds it: instruction issue and LDS latency of the table steps, not
@@ -17,16 +18,18 @@
 // each (row, token) pair in place, one token a lane and one row after another,
 // took 382 us for 256 rows of random JSON prefixes (about 110 distinct
 // states): a wave paid for its longest token and for every branch any of its
-// tokens took.  This way takes 45 us, about 27 us of it issue (13.3 M wave
-// instructions); 594 workgroups leave a few CUs with one more than the others.
-// Smaller workgroups even that out but repeat the tables and the search for
-// equal states: 128 tokens each took 55 us, four waves to 64 tokens 88 us.
+// tokens took.  This way takes 34 to 39 us from box to box, about 22 us of it
+// VALU issue (13.4 M wave instructions, and 7.1 M scalar, 1.2 M LDS ones); 594
+// workgroups leave a few CUs with one more than the others.  Smaller workgroups
+// even that out but repeat the tables and the search for equal states: 128
+// tokens each took 55 us, four waves to 64 tokens 88 us (where 256 tokens took
+// 45, before plain tokens passed in the walk).
 //
 // A mask set (tsm_json_masks_*) evaluates each distinct state of a call once
 // and keeps recent states' masks in device memory: one launch copies the rows
 // whose state the set holds, if any (and brings the new states into device
-// memory), another evaluates the new states, writing each into its slot and into every
-// row in that state.  The host keeps the index (state -> slot, least recently
+// memory), another evaluates the new states, writing each into its slot and
+// into every row in that state.  The host keeps the index (state -> slot, least recently
 // used out first), so no lookup waits for the GPU.
 #include <algorithm>
 #include <cstdarg>

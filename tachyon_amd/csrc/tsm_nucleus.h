@@ -44,7 +44,7 @@ constexpr uint32_t kNoBin = 0xFFFFFFFFu;
 constexpr uint32_t kNoRun = 0xFFFFFFFFu;
 constexpr uint32_t kBL = 4;         // bins per lane in a walk step
 
-// ---- LDS layout (above the re-read pass's per-tile history counts) ----------
+// ---- LDS layout (above the re-read pass's penalty table or counts) ----------
 constexpr uint32_t kOffE = kOffRank;
 constexpr uint32_t kOffECnt = kOffE;                     // u32[kNB] candidates per bin
 constexpr uint32_t kOffEMass = kOffECnt + kNB * 4;       // f64[kNB] approximate masses; after planning:

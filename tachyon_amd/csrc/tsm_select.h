@@ -3,8 +3,8 @@
 // L2 / MALL) and the exact finish of a ranked candidate list (the reference's
 // sequential f32 arithmetic).
 //
-// A re-read streams the row in 8192-id tiles and answers order-statistic
-// questions with 11-bit LDS histograms: select_kth gives the k-th element in
+// A re-read streams the row in tiles of 16,384 ids (row_blocks) and answers
+// order-statistic questions with 11-bit LDS histograms: select_kth gives the k-th element in
 // (value desc, id asc) order (radix).  When at most 1024 candidates remain
 // they are gathered, sorted and finished by exact_finalize, which reproduces
 // the CPU sampler's roundings; larger nucleus sets are finished by the value-
@@ -18,16 +18,18 @@ namespace tsm {
 // ---- LDS layout of the sampling workgroup (bytes) -----------------------------
 // Region A holds the streaming pass's history lookup (a bitmap of the ids in
 // the row's history and an open-addressing table of their counts) and, once
-// the stream is done, the finish's ranked lists and the re-read's per-tile
-// history counts.  The histograms, the candidate buffer, the penalized list
-// and the scalars have their own regions.
-constexpr uint32_t kReTile = 8192;         // ids per tile of a re-read pass
+// the stream is done, the finish's ranked lists and the re-read's table of
+// penalized ids (for longer histories, the history counts of a stretch of
+// kReTile ids).  The histograms, the candidate buffer, the penalized list and
+// the scalars have their own regions; a re-read keeps its bitmap of penalized
+// ids in the stream's histograms, which are read no more by then.
+constexpr uint32_t kReTile = 8192;         // ids of a counted stretch (half a tile of a re-read pass)
 constexpr uint32_t kBufCap = 6144;         // candidate buffer entries (y bits, id | flags)
 constexpr uint32_t kPenCap = 2048;         // penalized-id list entries (raw x bits, id)
 constexpr uint32_t kOffBitmap = 0;                              // u32[kBitmapWords]
 constexpr uint32_t kOffHashKey = kOffBitmap + kBitmapWords * 4;  // u32[kHashSlots]: id + 1, 0 = empty
 constexpr uint32_t kOffHashCnt = kOffHashKey + kHashSlots * 4;   // u32[kHashSlots]
-constexpr uint32_t kOffCnt = 0;                                  // u16 history counts of one re-read tile
+constexpr uint32_t kOffCnt = 0;                                  // re-read: u32[kPenSlots] table, or u16[kReTile] counts
 constexpr uint32_t kOffRank = kOffCnt + kReTile * 2;             // ry, rid, rp [kExactCap]
 constexpr uint32_t kOffGather = kOffRank + kExactCap * 12;       // rP, rq [kExactCap] | gcomp u64[kExactCap]
 constexpr uint32_t kRegionA = 65536;
@@ -39,7 +41,7 @@ constexpr uint32_t kOffMisc = kOffPen + kPenCap * 8;             // u32[64]
 constexpr uint32_t kOffMiscD = kOffMisc + 64 * 4;                // f64[32]
 constexpr uint32_t kOffTmp = kOffMiscD + 32 * 8;                 // u32[64] scan scratch
 constexpr uint32_t kSBins = 512;                                 // stream histogram bins per threshold
-constexpr uint32_t kOffSHist = kOffTmp + 64 * 4;                 // 2 x u32[kSBins]
+constexpr uint32_t kOffSHist = kOffTmp + 64 * 4;                 // 2 x u32[kSBins]; re-read: u32[kPenBitIds / 32] bitmap
 constexpr uint32_t kOffSeg = kOffSHist + 2 * kSBins * 4;         // stream counters (candidate groups)
 constexpr uint32_t kOffNanW = kOffSeg + 2 * (kBlock / kWave) * 4;  // per wave: met a NaN logit
 constexpr uint32_t kSmem = kOffNanW + (kBlock / kWave) * 4;
