@@ -9,7 +9,8 @@ pytestmark = pytest.mark.gpu
 
 def test_plain_tokens_cost_no_step_per_byte():
     """16 rows after a backslash, 4,000 tokens that begin with an escape's letter: 8 bytes long against 200 bytes
-    long, at most half as much time again.  (Stepped byte by byte the long ones took several times the short ones'.)"""
+    long, at most twice the time (launches of 10 us, which the host's own time moves; stepped byte by byte the long
+    ones took 68 us)."""
     import torch
 
     from tachyon_amd.constrain import DeviceVocab, HostVocab, JsonConstraint, json_mask, pack_states
@@ -38,4 +39,4 @@ def test_plain_tokens_cost_no_step_per_byte():
     us(8)
     short, long = us(8), us(200)
     print(f"8 bytes {short:.1f} us, 200 bytes {long:.1f} us", flush=True)
-    assert long < 1.5 * short
+    assert long < 2.0 * short
